@@ -448,6 +448,33 @@ int mhs_rmsnorm_bwd_f32(const float* dy, const float* x, const float* weight, co
                         const float* dres, float* dx, float* dweight, void* workspace,
                         size_t workspace_bytes, int64_t rows, int64_t cols, void* stream);
 
+/*
+ * fp32 matrix products of row-major operands (rows ld* apart), computed on the
+ * bf16 matrix cores from each value's three bf16 parts, with the error of an
+ * fp32 product:
+ *     MHS_GEMM_NT: c (m, n) = a (m, k) b (n, k)^T
+ *     MHS_GEMM_NN: c (m, n) = a (m, k) b (k, n)
+ *     MHS_GEMM_TN: c (m, n) = a (k, m)^T b (k, n)
+ * With accumulate, c +=. They are the products of the block's projections, of
+ * the tied head and of their gradients (nn.Linear at mamba_metal/model.py:
+ * 172-183, :197-200, :256, :294). Operands contiguous in k (a of NT and NN, b
+ * of NT) need k and their row stride to be multiples of 4 and a 16-byte
+ * aligned pointer. Infinities and NaN come out as in plain fp32. Deterministic.
+ *
+ * mhs_gemm_workspace_bytes: the device workspace (256-byte aligned) of a
+ * product, 0 for none, -1 for invalid sizes. With a workspace, c must be
+ * 16-byte aligned and ldc a multiple of 4. mhs_gemm_preferred: 1 where the
+ * product is faster than a BLAS library's fp32 one (large products), else 0.
+ */
+#define MHS_GEMM_NT 0
+#define MHS_GEMM_NN 1
+#define MHS_GEMM_TN 2
+int mhs_gemm_preferred(int64_t m, int64_t n, int64_t k);
+int64_t mhs_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int mhs_gemm_f32(int form, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
+                 int64_t ldc, int64_t m, int64_t n, int64_t k, int accumulate, void* workspace,
+                 size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -36,7 +36,8 @@ EXPORTED_SYMBOLS = (
     "mhs_deterministic",
     "mhs_scan_bwd_reduction", "mhs_xent_fwd_f32", "mhs_xent_bwd_f32",
     "mhs_rmsnorm_fwd_f32", "mhs_rmsnorm_bwd_workspace_bytes", "mhs_rmsnorm_bwd_f32",
-    "mhs_add_rmsnorm_fwd_f32",
+    "mhs_add_rmsnorm_fwd_f32", "mhs_gemm_preferred",
+    "mhs_gemm_workspace_bytes", "mhs_gemm_f32",
 )
 
 # Size of the static device scratch of mhs_scan_fwd_noalloc_f32 (the header's
@@ -143,6 +144,13 @@ def library() -> ctypes.CDLL:
             lib.mhs_rmsnorm_bwd_workspace_bytes.argtypes = [_I64] * 2
             lib.mhs_rmsnorm_bwd_f32.restype = ctypes.c_int
             lib.mhs_rmsnorm_bwd_f32.argtypes = [_P] * 8 + [ctypes.c_size_t] + [_I64] * 2 + [_P]
+            lib.mhs_gemm_preferred.restype = ctypes.c_int
+            lib.mhs_gemm_preferred.argtypes = [_I64] * 3
+            lib.mhs_gemm_workspace_bytes.restype = _I64
+            lib.mhs_gemm_workspace_bytes.argtypes = [_I64] * 3
+            lib.mhs_gemm_f32.restype = ctypes.c_int
+            lib.mhs_gemm_f32.argtypes = ([ctypes.c_int] + [_P, _I64] * 3 + [_I64] * 3
+                                         + [ctypes.c_int, _P, ctypes.c_size_t, _P])
             _lib = lib
     return _lib
 
@@ -1038,3 +1046,100 @@ rmsnorm_bwd = _register(
 @rmsnorm_bwd.register_fake
 def _rmsnorm_bwd_fake(dy, x, weight, rstd, dres):
     return torch.empty_like(x), torch.empty_like(weight)
+
+
+# ---------------------------------------------------------- matrix products
+
+GEMM_NT, GEMM_NN, GEMM_TN = 0, 1, 2
+
+
+def _gemm_sizes(a: torch.Tensor, b: torch.Tensor, form: int) -> tuple[int, int, int]:
+    """(m, n, k) of a b^T (GEMM_NT), a b (GEMM_NN) or a^T b (GEMM_TN)."""
+    m, k = a.shape if form != GEMM_TN else (a.shape[1], a.shape[0])
+    return m, b.shape[0] if form == GEMM_NT else b.shape[1], k
+
+
+@torch.compiler.assume_constant_result
+def gemm_preferred(m: int, n: int, k: int) -> bool:
+    """Whether the HIP product is the faster at these sizes (else the
+    framework's)."""
+    return library().mhs_gemm_preferred(m, n, k) != 0
+
+
+def _rows2(t: torch.Tensor, k_major: bool) -> bool:
+    """Whether the kernel reads the 2-D operand in place."""
+    ld = t.stride(0)
+    return (t.stride(1) == 1 and ld >= t.shape[1] and ld < 1 << 22
+            and (not k_major or (t.shape[1] % 4 == 0 and ld % 4 == 0 and t.data_ptr() % 16 == 0)))
+
+
+def _gemm_into(a: torch.Tensor, b: torch.Tensor, form: int, out: torch.Tensor,
+               accumulate: bool) -> bool:
+    """The HIP product into out (2-D, rows contiguous); False where it does not
+    take the operands or the framework's is the faster."""
+    m, n, k = _gemm_sizes(a, b, form)
+    if not (a.is_cuda and a.dtype == b.dtype == out.dtype == torch.float32 and m and n and k
+            and _rows2(a, form != GEMM_TN) and _rows2(b, form == GEMM_NT)):
+        return False
+    lib = library()
+    if not lib.mhs_gemm_preferred(m, n, k):
+        return False
+    nbytes = int(lib.mhs_gemm_workspace_bytes(m, n, k))
+    if nbytes and (out.stride(0) % 4 or out.data_ptr() % 16):
+        return False
+    with _on(a.device):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=a.device) if nbytes else None
+        rc = lib.mhs_gemm_f32(form, _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(out),
+                              out.stride(0), m, n, k, accumulate, _ptr(ws), nbytes,
+                              _stream(a.device))
+    _check(rc, "mhs_gemm_f32")
+    return True
+
+
+def _mm(a: torch.Tensor, b: torch.Tensor, form: int) -> torch.Tensor:
+    """The framework's product."""
+    if form == GEMM_NT:
+        return torch.mm(a, b.t())
+    return torch.mm(a, b) if form == GEMM_NN else torch.mm(a.t(), b)
+
+
+def _gemm_impl(a: torch.Tensor, b: torch.Tensor, form: int) -> torch.Tensor:
+    """a b^T (GEMM_NT), a b (GEMM_NN) or a^T b (GEMM_TN) of 2-D fp32 tensors."""
+    m, n, _ = _gemm_sizes(a, b, form)
+    out = a.new_empty((m, n))
+    return out if _gemm_into(a, b, form, out, False) else _mm(a, b, form)
+
+
+def _check_gemm(what: str, a, b, form, out=None) -> None:
+    _on_one_device(what, a, b, out)
+    _fp32(what, a=a, b=b, out=out)
+    _need(form in (GEMM_NT, GEMM_NN, GEMM_TN) and a.dim() == 2 and b.dim() == 2, what,
+          f"a and b must be 2-D and form 0..2; got {tuple(a.shape)}, {tuple(b.shape)}, {form}")
+    m, n, k = _gemm_sizes(a, b, form)
+    _need(k == (b.shape[1] if form == GEMM_NT else b.shape[0]), what,
+          f"sizes do not match: {tuple(a.shape)}, {tuple(b.shape)}, form {form}")
+    _shaped(what, "out", out, (m, n))
+    _dense(what, out=out)
+
+
+gemm = _register("gemm", _gemm_impl, (), lambda a, b, form: _check_gemm("gemm", a, b, form))
+
+
+@gemm.register_fake
+def _gemm_fake(a, b, form):
+    return a.new_empty(_gemm_sizes(a, b, form)[:2])
+
+
+def _gemm_add_impl(out: torch.Tensor, a: torch.Tensor, b: torch.Tensor, form: int) -> None:
+    """out += the product of gemm; out contiguous."""
+    if not _gemm_into(a, b, form, out, True):
+        out.add_(_mm(a, b, form)) if form != GEMM_NN else out.addmm_(a, b)
+
+
+gemm_add = _register("gemm_add", _gemm_add_impl, ("out",),
+                     lambda out, a, b, form: _check_gemm("gemm_add", a, b, form, out))
+
+
+@gemm_add.register_fake
+def _gemm_add_fake(out, a, b, form):
+    return None

@@ -165,7 +165,8 @@ class MambaInnerHIP(torch.autograd.Function):
         xc = _native.dispatch("conv1d_silu_fwd")(x, w2, cb)
         w_proj = torch.cat([w_dt, w_b, w_c], 0)
         bias = b_dt.contiguous()
-        proj = torch.mm(xc.view(-1, d), w_proj.t()).view(bt, t_len, d + 2 * n)
+        proj = _native.dispatch("gemm")(xc.view(-1, d), w_proj,
+                                        _native.GEMM_NT).view(bt, t_len, d + 2 * n)
         need_grad = any(ctx.needs_input_grad)
         y, ckpt, _ = _native.dispatch("scan_gated_fwd")(
             xc, proj[..., :d], a_raw, proj[..., d:d + n], proj[..., d + n:], float(dt_min),
@@ -191,8 +192,9 @@ class MambaInnerHIP(torch.autograd.Function):
             xc, proj[..., :d], a_raw, proj[..., d:d + n], proj[..., d + n:], ctx.gate[0],
             ctx.gate[1], dy, None, ckpt, ctx.chunk, dproj, bias)
         dp2 = dproj.view(-1, d + 2 * n)
-        dxc.view(-1, d).addmm_(dp2, w_proj)            # + the projections' input gradient
-        dw = dp2.t().mm(xc.view(-1, d))
+        # + the projections' input gradient
+        _native.dispatch("gemm_add")(dxc.view(-1, d), dp2, w_proj, _native.GEMM_NN)
+        dw = _native.dispatch("gemm")(dp2, xc.view(-1, d), _native.GEMM_TN)
         dcw, dcb = _native.dispatch("conv1d_silu_bwd_into")(xz[..., :d], w2, cb, dxc,
                                                             dxz[..., :d])
         return (dxz, dcw.reshape(ctx.conv_shape), dcb, dw[:d], db_dt, dw[d:d + n],

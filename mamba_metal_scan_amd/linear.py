@@ -1,0 +1,63 @@
+"""Bias-free fp32 linear layers of the model on the HIP matrix products.
+
+The reference's ``in_proj``, ``out_proj`` and tied head are ``nn.Linear``
+without a bias (mamba_metal/model.py:172, :183, :294). ``linear`` computes
+``x W^T`` and its gradients ``dy W`` and ``dy^T x`` with the library's
+products (three bf16 parts per fp32 value on the bf16 matrix cores), each
+where it is the faster, else with the framework's.
+"""
+from __future__ import annotations
+
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from . import _native
+from ._native import GEMM_NN, GEMM_NT, GEMM_TN, dispatch
+
+
+class LinearHIP(torch.autograd.Function):
+    """x (rows, in) W (out, in)^T, fp32."""
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        ctx.save_for_backward(x, weight)
+        return dispatch("gemm")(x, weight, GEMM_NT)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        dy = dy.contiguous()
+        if torch.is_grad_enabled():   # create_graph: products that can be differentiated
+            return (dy.mm(weight) if ctx.needs_input_grad[0] else None,
+                    dy.t().mm(x) if ctx.needs_input_grad[1] else None)
+        dx = dispatch("gemm")(dy, weight, GEMM_NN) if ctx.needs_input_grad[0] else None
+        dw = dispatch("gemm")(dy, x, GEMM_TN) if ctx.needs_input_grad[1] else None
+        return dx, dw
+
+
+def no_hooks(m: nn.Module) -> bool:
+    """Whether neither m nor the module-global registries hold forward or
+    backward hooks."""
+    g = nn.modules.module
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks or g._global_forward_hooks
+                or g._global_forward_pre_hooks or g._global_backward_hooks
+                or g._global_backward_pre_hooks)
+
+
+def linear(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """mod(x), through the HIP products where mod is a plain bias-free
+    nn.Linear (no subclass, no hooks), x and its weight are fp32 on one ROCm
+    device outside autocast, and the product is large enough to be the faster
+    there (smaller ones keep the framework's call and its lower overhead)."""
+    if (type(mod) is nn.Linear and mod.bias is None and x.is_cuda and x.dtype == torch.float32
+            and torch.version.hip is not None and not torch.is_autocast_enabled()):
+        w = mod.weight
+        k = x.shape[-1]
+        if (k > 0 and w.dtype == torch.float32 and w.device == x.device and w.shape[1] == k
+                and w.is_contiguous() and no_hooks(mod)
+                and _native.gemm_preferred(x.numel() // k, w.shape[0], k)):
+            x2 = x.reshape(-1, k)
+            return LinearHIP.apply(x2, w).view(*x.shape[:-1], w.shape[0])
+    return mod(x)

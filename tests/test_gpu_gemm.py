@@ -1,0 +1,118 @@
+"""GPU parity of the fp32 matrix products on the bf16 matrix cores with
+float64, at the edges of their tiles (128 x 128, 16 deep) and of the split
+over k.
+
+Bar, per element: |got - ref| <= (6 K / 16 + S + 8) 2^-23 sum_k |a_k b_k|: the
+product of a k tile is six additions to the sum, each rounding (or
+truncating) by at most 2^-23 of the running sum, which sum_k |a_k b_k| bounds;
+S more additions sum the splits, and the dropped parts and the parts' own
+roundings stay below the 8.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from mamba_metal_scan_amd import _native
+from mamba_metal_scan_amd._native import GEMM_NN, GEMM_NT, GEMM_TN
+from mamba_metal_scan_amd.linear import LinearHIP
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+FORMS = {"nt": GEMM_NT, "nn": GEMM_NN, "tn": GEMM_TN}
+
+
+def _operands(form, m, n, k, seed=0, pad=0):
+    g = torch.Generator().manual_seed(seed + m * 7 + n * 3 + k)
+
+    def mat(r, c):
+        return torch.randn(r, c + pad, generator=g).to(DEV)[:, :c]
+    return (mat(k, m) if form == GEMM_TN else mat(m, k),
+            mat(n, k) if form == GEMM_NT else mat(k, n))
+
+
+def _ref(a, b, form):
+    a = a.t() if form == GEMM_TN else a
+    return a @ (b.t() if form == GEMM_NT else b)
+
+
+def _call(a, b, form, out, accumulate=False):
+    """The C entry at any size (the Python layer sends small ones elsewhere)."""
+    lib = _native.library()
+    m, n, k = _native._gemm_sizes(a, b, form)
+    need = lib.mhs_gemm_workspace_bytes(m, n, k)
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=DEV)
+    rc = lib.mhs_gemm_f32(form, a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+                          out.data_ptr(), out.stride(0), m, n, k, accumulate, ws.data_ptr(),
+                          need, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, lib.mhs_last_error()
+    torch.cuda.synchronize()
+    return need
+
+
+def _assert_bounded(got, a, b, form, k, extra=0):
+    ref = _ref(a.double(), b.double(), form)
+    bound = (6 * k / 16 + 32 + 8) * 2.0 ** -23 * _ref(a.double().abs(), b.double().abs(), form)
+    bad = ((got.double() - extra - ref).abs() > bound + 2.0 ** -22 * abs(extra)).sum().item()
+    assert bad == 0, f"{bad} elements off"
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("m,n,k", [(1, 4, 4), (128, 128, 16), (129, 132, 20), (127, 260, 1432),
+                                   (300, 8, 36), (257, 128, 8192)])
+def test_products_match_float64(form, m, n, k):
+    print(f"[case] gemm {form} {m}x{n}x{k}", flush=True)
+    f = FORMS[form]
+    for pad in (0, 4):
+        a, b = _operands(f, m, n, k, pad=pad)
+        out = torch.full((m, n), float("nan"), device=DEV)
+        _call(a, b, f, out)
+        _assert_bounded(out, a, b, f, k)
+        _call(a, b, f, out.fill_(0.5), accumulate=True)
+        _assert_bounded(out, a, b, f, k, extra=0.5)
+
+
+@pytest.mark.parametrize("form,m,n,k", [("nn", 33, 7, 64), ("tn", 33, 7, 37), ("nt", 33, 7, 64)])
+def test_widths_that_are_no_multiple_of_four(form, m, n, k):
+    f = FORMS[form]
+    a, b = _operands(f, m, n, k)
+    out = torch.full((m, n), float("nan"), device=DEV)
+    assert _call(a, b, f, out) == 0   # never split
+    _assert_bounded(out, a, b, f, k)
+
+
+def test_infinities_and_nan_come_out_as_in_fp32():
+    a, b = _operands(GEMM_NT, 200, 140, 64)
+    a[3, 5], a[7, 9], b[11, 2], a[20, 1] = float("inf"), float("nan"), -float("inf"), 3.4e38
+    a[21], b[30] = 1e30, 1e30
+    ref = _ref(a, b, GEMM_NT)
+    out = torch.empty(200, 140, device=DEV)
+    _call(a, b, GEMM_NT, out)
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(torch.isinf(out), inf) and torch.equal(out[inf], ref[inf])
+
+
+@pytest.mark.parametrize("scale", [1e-12, 1e-19, 1e15])
+def test_scales(scale):
+    a, b = (v * scale for v in _operands(GEMM_NT, 130, 128, 256))
+    out = torch.empty(130, 128, device=DEV)
+    _call(a, b, GEMM_NT, out)
+    _assert_bounded(out, a, b, GEMM_NT, 256)
+
+
+def test_linear_gradients():
+    """A layer large enough for the HIP products in every direction."""
+    rows, k, n = 2048, 640, 1464
+    assert _native.gemm_preferred(rows, n, k)
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn(rows, k, generator=g).to(DEV).requires_grad_()
+    w = torch.randn(n, k, generator=g).to(DEV).requires_grad_()
+    dy = torch.randn(rows, n, generator=g).to(DEV)
+    y = LinearHIP.apply(x, w)
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    _assert_bounded(y.detach(), x.detach(), w.detach(), GEMM_NT, k)
+    _assert_bounded(dx, dy, w.detach(), GEMM_NN, n)
+    _assert_bounded(dw, dy, x.detach(), GEMM_TN, rows)
