@@ -475,6 +475,39 @@ int mhs_gemm_f32(int form, const float* a, int64_t lda, const float* b, int64_t 
                  int64_t ldc, int64_t m, int64_t n, int64_t k, int accumulate, void* workspace,
                  size_t workspace_bytes, void* stream);
 
+/*
+ * One recurrent token of the whole model, fp32 (the step of the reference's
+ * MambaBlock, mamba_metal/model.py:228-256, through every block, the final
+ * norm and the head, :289-298): per block, in order, the RMSNorm, in_proj, the
+ * causal conv's step with SiLU, the dt / B / C projections with the dt gate,
+ * the state's update, the output gate and out_proj with the residual; then
+ * logits = head (vocab, d_model) of the normalised result.
+ * x (batch, d_model): the token's embeddings (read only). Per layer: the
+ * weights as nn.Linear / nn.Conv1d hold them, contiguous; h (batch, d_inner,
+ * d_state), advanced in place; conv, the last conv_taps - 1 inputs of the conv
+ * (batch, d_inner, conv_taps - 1) with the strides conv_s* (elements),
+ * conv_next the window after this token, contiguous, not conv itself. d_model
+ * and d_inner are multiples of 4; the linear weights, the norms and x are
+ * 16-byte aligned; the workspace is 256-byte aligned. Every pointer is used by
+ * this call's launches only.
+ */
+typedef struct mhs_decode_layer {
+  const float *norm_weight, *in_proj, *conv_weight, *conv_bias, *dt_proj, *dt_bias, *A, *B_proj,
+      *C_proj, *D_skip, *out_proj;
+  float* h;
+  const float* conv;
+  int64_t conv_sb, conv_sd, conv_sk;
+  float* conv_next;
+  float eps, dt_min, dt_max, unused;
+} mhs_decode_layer;
+size_t mhs_decode_workspace_bytes(int64_t batch, int64_t d_model, int64_t d_inner,
+                                  int64_t d_state);
+int mhs_decode_f32(const mhs_decode_layer* layers, int64_t n_layers, const float* x,
+                   const float* norm_weight, float eps, const float* head, float* logits,
+                   int64_t batch, int64_t d_model, int64_t d_inner, int64_t d_state,
+                   int64_t conv_taps, int64_t vocab, void* workspace, size_t workspace_bytes,
+                   void* stream);
+
 #ifdef __cplusplus
 }
 #endif

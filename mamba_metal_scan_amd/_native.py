@@ -37,7 +37,8 @@ EXPORTED_SYMBOLS = (
     "mhs_scan_bwd_reduction", "mhs_xent_fwd_f32", "mhs_xent_bwd_f32",
     "mhs_rmsnorm_fwd_f32", "mhs_rmsnorm_bwd_workspace_bytes", "mhs_rmsnorm_bwd_f32",
     "mhs_add_rmsnorm_fwd_f32", "mhs_gemm_preferred",
-    "mhs_gemm_workspace_bytes", "mhs_gemm_f32",
+    "mhs_gemm_workspace_bytes", "mhs_gemm_f32", "mhs_decode_workspace_bytes",
+    "mhs_decode_f32",
 )
 
 # Size of the static device scratch of mhs_scan_fwd_noalloc_f32 (the header's
@@ -151,6 +152,11 @@ def library() -> ctypes.CDLL:
             lib.mhs_gemm_f32.restype = ctypes.c_int
             lib.mhs_gemm_f32.argtypes = ([ctypes.c_int] + [_P, _I64] * 3 + [_I64] * 3
                                          + [ctypes.c_int, _P, ctypes.c_size_t, _P])
+            lib.mhs_decode_workspace_bytes.restype = ctypes.c_size_t
+            lib.mhs_decode_workspace_bytes.argtypes = [_I64] * 4
+            lib.mhs_decode_f32.restype = ctypes.c_int
+            lib.mhs_decode_f32.argtypes = ([ctypes.c_char_p, _I64, _P, _P, _F32, _P, _P]
+                                           + [_I64] * 6 + [_P, ctypes.c_size_t, _P])
             _lib = lib
     return _lib
 

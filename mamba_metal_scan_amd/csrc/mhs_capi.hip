@@ -19,6 +19,7 @@
 #include "mamba_hip_scan.h"
 #include "mhs_bwd.hpp"
 #include "mhs_conv.hpp"
+#include "mhs_decode.hpp"
 #include "mhs_fwd.hpp"
 #include "mhs_gate.hpp"
 #include "mhs_gemm.hpp"
@@ -1594,6 +1595,153 @@ int mhs_gemm_f32(int form, const float* a, int64_t lda, const float* b, int64_t 
                      dim3(256), 0, s, g.C, c, p.splits, (long long)m, (int)(n / 4),
                      (long long)(ldc / 4), accumulate);
   return check_launch("matrix product reduction kernel");
+}
+
+}  // extern "C"
+
+// ------------------------------------------------------- one token, whole model
+
+namespace {
+
+// Batch rows per wave: all of a small batch, else 8 at a time (the weights'
+// rows then come from the caches again).
+template <int KIND, int RW>
+int launch_decode(const mhs::DecodeArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.rows + 4 * RW - 1) / (4 * RW))), block(256);
+  if (a.batch == 1)
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 1, RW>), grid, block, 0, s, a);
+  else if (a.batch == 2)
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 2, RW>), grid, block, 0, s, a);
+  else if (a.batch <= 4)
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 4, RW>), grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 8, RW>), grid, block, 0, s, a);
+  return check_launch("decode product kernel");
+}
+
+// Workspace of a token: xc, z, dt, g (batch, D), B and C (batch, N each), x
+// (batch, d_model), each 16-byte aligned.
+struct DecodeWs {
+  size_t xc, z, dt, g, bc, x, total;
+};
+
+DecodeWs decode_ws(int64_t batch, int64_t d_model, int64_t D, int64_t N) {
+  DecodeWs w;
+  const size_t row = round_up((size_t)batch * D * 4, 256);
+  w.xc = 0;
+  w.z = row;
+  w.dt = 2 * row;
+  w.g = 3 * row;
+  w.bc = 4 * row;
+  w.x = w.bc + round_up((size_t)2 * batch * N * 4, 256);
+  w.total = w.x + round_up((size_t)batch * d_model * 4, 256);
+  return w;
+}
+
+int check_decode(int64_t batch, int64_t d_model, int64_t d_inner, int64_t d_state, int64_t taps,
+                 int64_t vocab) {
+  if (batch < 1 || batch > 65535 || d_model < 4 || d_inner < 4 || d_state < 1 || vocab < 1 ||
+      d_model % 4 || d_inner % 4 || d_model > (1 << 20) || d_inner > (1 << 20) ||
+      d_state > MHS_MAX_DSTATE || vocab > (1 << 28) || taps < 2 || taps > mhs::kConvMaxK)
+    return fail(MHS_EINVAL, "unsupported sizes: batch %lld d_model %lld d_inner %lld (multiples "
+                "of 4) d_state %lld conv taps %lld vocab %lld", (long long)batch,
+                (long long)d_model, (long long)d_inner, (long long)d_state, (long long)taps,
+                (long long)vocab);
+  return MHS_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t mhs_decode_workspace_bytes(int64_t batch, int64_t d_model, int64_t d_inner,
+                                  int64_t d_state) {
+  if (check_decode(batch, d_model, d_inner, d_state, 2, 1)) return 0;
+  return decode_ws(batch, d_model, d_inner, d_state).total;
+}
+
+int mhs_decode_f32(const mhs_decode_layer* layers, int64_t n_layers, const float* x,
+                   const float* norm_weight, float eps, const float* head, float* logits,
+                   int64_t batch, int64_t d_model, int64_t d_inner, int64_t d_state,
+                   int64_t conv_taps, int64_t vocab, void* workspace, size_t workspace_bytes,
+                   void* stream) {
+  g_err[0] = '\0';
+  int rc = check_decode(batch, d_model, d_inner, d_state, conv_taps, vocab);
+  if (rc) return rc;
+  if ((n_layers > 0 && !layers) || n_layers < 0 || !x || !norm_weight || !head || !logits ||
+      !workspace)
+    return fail(MHS_EINVAL, "null pointer argument");
+  const DecodeWs w = decode_ws(batch, d_model, d_inner, d_state);
+  if (workspace_bytes < w.total)
+    return fail(MHS_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, w.total);
+  if (reinterpret_cast<uintptr_t>(workspace) & 255u)
+    return fail(MHS_EINVAL, "workspace must be 256-byte aligned");
+  for (const void* q : {(const void*)x, (const void*)norm_weight, (const void*)head})
+    if (!aligned16(q)) return fail(MHS_EINVAL, "device pointers must be 16-byte aligned");
+  for (int64_t l = 0; l < n_layers; ++l) {
+    const mhs_decode_layer& p = layers[l];
+    for (const void* q : {(const void*)p.norm_weight, (const void*)p.in_proj,
+                          (const void*)p.conv_weight, (const void*)p.conv_bias,
+                          (const void*)p.dt_proj, (const void*)p.dt_bias, (const void*)p.A,
+                          (const void*)p.B_proj, (const void*)p.C_proj, (const void*)p.D_skip,
+                          (const void*)p.out_proj, (const void*)p.h, (const void*)p.conv,
+                          (const void*)p.conv_next})
+      if (!q) return fail(MHS_EINVAL, "null pointer in layer %lld", (long long)l);
+    for (const void* q : {(const void*)p.norm_weight, (const void*)p.in_proj,
+                          (const void*)p.dt_proj, (const void*)p.B_proj, (const void*)p.C_proj,
+                          (const void*)p.out_proj})
+      if (!aligned16(q)) return fail(MHS_EINVAL, "device pointers must be 16-byte aligned");
+    if (p.conv_next == p.conv) return fail(MHS_EINVAL, "conv_next may not alias conv");
+    Gate g;
+    rc = check_gate(p.dt_min, p.dt_max, g);
+    if (rc) return rc;
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  auto at = [&](size_t off) { return reinterpret_cast<float*>(ws + off); };
+  float *xc = at(w.xc), *z = at(w.z), *dt = at(w.dt), *g = at(w.g), *bc = at(w.bc);
+  const int nb = (int)batch, D = (int)d_inner, N = (int)d_state, M = (int)d_model;
+  const float* xin = x;
+  for (int64_t l = 0; l < n_layers; ++l) {
+    const mhs_decode_layer& p = layers[l];
+    mhs::DecodeArgs a{};
+    a.batch = nb;
+    a.D = D;
+    a.N = N;
+    a.x = xin; a.w = p.in_proj; a.K = M; a.rows = 2 * D;
+    a.norm_w = p.norm_weight; a.eps = p.eps;
+    a.out = xc; a.out2 = z;
+    a.conv_w = p.conv_weight; a.conv_b = p.conv_bias; a.conv = p.conv;
+    a.conv_sb = p.conv_sb; a.conv_sd = p.conv_sd; a.conv_sk = p.conv_sk;
+    a.conv_next = p.conv_next; a.taps = (int)conv_taps;
+    rc = launch_decode<mhs::kDecIn, 2>(a, s);
+    if (rc) return rc;
+    a.x = xc; a.w = p.dt_proj; a.w_b = p.B_proj; a.w_c = p.C_proj; a.K = D; a.rows = D + 2 * N;
+    a.out = dt; a.out2 = bc; a.bias = p.dt_bias;
+    a.dt_lo = p.dt_min; a.dt_span = p.dt_max - p.dt_min;
+    rc = launch_decode<mhs::kDecProj, 1>(a, s);
+    if (rc) return rc;
+    const long long ch = batch * d_inner;
+    if (N >= 4)
+      hipLaunchKernelGGL(mhs::decode_state_kernel<4>, dim3((unsigned)((4 * ch + 255) / 256)),
+                         dim3(256), 0, s, p.h, xc, dt, p.A, bc, bc + (size_t)nb * N, p.D_skip, z,
+                         g, nb, D, N);
+    else
+      hipLaunchKernelGGL(mhs::decode_state_kernel<1>, dim3((unsigned)((ch + 255) / 256)),
+                         dim3(256), 0, s, p.h, xc, dt, p.A, bc, bc + (size_t)nb * N, p.D_skip, z,
+                         g, nb, D, N);
+    rc = check_launch("decode state kernel");
+    if (rc) return rc;
+    a.x = g; a.w = p.out_proj; a.K = D; a.rows = M; a.out = at(w.x); a.res = xin;
+    rc = launch_decode<mhs::kDecOut, 1>(a, s);
+    if (rc) return rc;
+    xin = at(w.x);   // updated in place by the later blocks
+  }
+  mhs::DecodeArgs a{};
+  a.batch = nb;
+  a.x = xin; a.w = head; a.K = M; a.rows = (int)vocab;
+  a.norm_w = norm_weight; a.eps = eps; a.out = logits;
+  return launch_decode<mhs::kDecHead, 4>(a, s);
 }
 
 }  // extern "C"

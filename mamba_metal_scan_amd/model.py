@@ -39,6 +39,7 @@ import torch.nn.functional as F
 
 from ._native import rmsnorm_supported
 from .conv import conv1d_silu
+from .decode import decode_step
 from .fused import mamba_inner, out_gate, selective_scan_gated
 from .linear import linear, no_hooks
 from .norm import add_rms_norm, rms_norm, rms_norm_residual
@@ -356,11 +357,8 @@ class TinyMamba(nn.Module):
         elif isinstance(m, nn.Embedding):
             nn.init.normal_(m.weight, mean=0.0, std=0.02)
 
-    def forward(self, idx, targets=None, cache=None):
-        if cache is not None and "blocks" not in cache:
-            cache["blocks"] = [{} for _ in self.blocks]
-        x = self.tok(idx)
-        caches = cache["blocks"] if cache is not None else [None] * len(self.blocks)
+    def _hidden(self, x, caches):
+        """The final norm's output for the embedded tokens x."""
         if self.ln_f.uses_hip(x) and all(_plain_block(b) and b.norm.uses_hip(x)
                                          for b in self.blocks):
             # The HIP norms: each block's residual add goes into the next norm's
@@ -376,13 +374,29 @@ class TinyMamba(nn.Module):
                     x, h = add_rms_norm(x, delta, block.norm.weight, block.norm.eps)
                 # (under autocast out_proj yields bf16: widened exactly, as x + delta would)
                 delta = block.mix(h, bc).to(x.dtype)
-            h = (add_rms_norm(x, delta, self.ln_f.weight, self.ln_f.eps)[1] if delta is not None
-                 else self.ln_f(x))
-        else:
-            for block, bc in zip(self.blocks, caches):
-                x = block(x, bc)
-            h = self.ln_f(x)
-        logits = self.head(h) if self.cfg.scan_impl == "torch" else linear(self.head, h)
+            return (add_rms_norm(x, delta, self.ln_f.weight, self.ln_f.eps)[1]
+                    if delta is not None else self.ln_f(x))
+        for block, bc in zip(self.blocks, caches):
+            x = block(x, bc)
+        return self.ln_f(x)
+
+    def _token(self, x, cache):
+        """The logits of one embedded token per sequence against the cache as
+        one native call, or None where that does not apply (see decode_step)."""
+        if (torch.is_grad_enabled() or self.cfg.scan_impl == "torch" or not _hip_device(x)
+                or not all(_plain_block(b) for b in self.blocks)):
+            return None
+        return decode_step(self, x, cache)
+
+    def forward(self, idx, targets=None, cache=None):
+        if cache is not None and "blocks" not in cache:
+            cache["blocks"] = [{} for _ in self.blocks]
+        x = self.tok(idx)
+        caches = cache["blocks"] if cache is not None else [None] * len(self.blocks)
+        logits = self._token(x, cache) if cache is not None and idx.shape[1] == 1 else None
+        if logits is None:
+            h = self._hidden(x, caches)
+            logits = self.head(h) if self.cfg.scan_impl == "torch" else linear(self.head, h)
         loss = None
         if targets is not None:
             flat, tflat = logits.reshape(-1, logits.size(-1)), targets.reshape(-1)

@@ -1,0 +1,122 @@
+"""GPU parity of the native one-token step of a TinyMamba (mhs_decode_f32):
+logits, states and conv windows against the float64 step of the torch model
+(scan_impl 'torch', the reference's own update, mamba_metal/model.py:228-256),
+over several tokens.
+
+Bar: 1e-4 max relative per tensor, the build's parity bar.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import assert_close
+from mamba_metal_scan_amd import decode
+from mamba_metal_scan_amd.model import MambaConfig, TinyMamba
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _models(**over):
+    kw = dict(vocab_size=203, d_model=64, n_layers=2, d_ff=128, max_seq_len=64, d_state=16,
+              d_conv=4)
+    kw.update(over)
+    torch.manual_seed(3)
+    hip = TinyMamba(MambaConfig(scan_impl="hip", **kw))
+    with torch.no_grad():   # not the initial zeros and ones
+        for b in hip.blocks:
+            b.dt_proj.bias.normal_()
+            b.D_skip.normal_()
+            b.norm.weight.normal_(1.0, 0.1)
+        hip.ln_f.weight.normal_(1.0, 0.1)
+    ref = TinyMamba(MambaConfig(scan_impl="torch", **kw)).double()
+    ref.load_state_dict({k: v.double() for k, v in hip.state_dict().items()})
+    return hip.to(DEV), ref
+
+
+def _native_calls(monkeypatch):
+    seen = []
+    real = decode.decode_step
+
+    def spy(*args):
+        out = real(*args)
+        seen.append(out is not None)
+        return out
+    monkeypatch.setattr("mamba_metal_scan_amd.model.decode_step", spy)
+    return seen
+
+
+# Batches around the kernels' 1, 2, 4 and 8 rows; widths whose K / 4 is below,
+# at and above one pass (128 lanes' loads); states of the 4-lane and the
+# 1-lane kernel, odd ones; the shortest and longest conv.
+@pytest.mark.parametrize("batch,over", [
+    (1, {}), (2, dict(d_model=128, d_inner=516)), (3, dict(d_state=5)), (4, dict(d_state=64)),
+    (5, dict(d_state=3, d_conv=2)), (8, dict(d_model=512, d_inner=512, d_conv=8)),
+    (9, dict(d_state=1, vocab_size=17)), (17, dict(d_model=516, d_inner=4, n_layers=1))])
+def test_token_matches_float64(monkeypatch, batch, over):
+    print(f"[case] decode batch {batch} {over}", flush=True)
+    hip, ref = _models(**over)
+    seen = _native_calls(monkeypatch)
+    vocab = hip.cfg.vocab_size
+    idx = torch.randint(0, vocab, (batch, 9), generator=torch.Generator().manual_seed(batch))
+    ch, cr = {}, {}
+    with torch.no_grad():
+        hip(idx[:, :6].to(DEV), cache=ch)
+        ref(idx[:, :6], cache=cr)
+        for t in range(6, 9):
+            lh, _ = hip(idx[:, t:t + 1].to(DEV), cache=ch)
+            lr, _ = ref(idx[:, t:t + 1], cache=cr)
+            torch.cuda.synchronize()
+            assert_close("logits", lh, lr)
+            for bh, br in zip(ch["blocks"], cr["blocks"]):
+                assert_close("h", bh["h"], br["h"])
+                assert_close("conv", bh["conv"], br["conv"])
+    assert seen == [True] * 3
+
+
+def test_other_forms_take_the_general_step(monkeypatch):
+    """A hook inside a block and autograd keep the module calls, with the same
+    results; so does autocast, which their step kernel refuses."""
+    hip, ref = _models()
+    seen = _native_calls(monkeypatch)
+    idx = torch.randint(0, 203, (2, 8), generator=torch.Generator().manual_seed(1)).to(DEV)
+
+    def step(ctx, prepare=lambda: None):
+        cache = {}
+        with torch.no_grad():
+            hip(idx[:, :-1], cache=cache)
+        prepare()
+        with ctx:
+            return hip(idx[:, -1:], cache=cache)[0].detach().float()
+
+    want = step(torch.no_grad())
+    assert seen == [True]
+    assert_close("autograd", step(torch.enable_grad()), want)
+    assert len(seen) == 1    # not asked
+    hook = []
+    handles = []
+    got = step(torch.no_grad(), lambda: handles.append(
+        hip.blocks[1].in_proj.register_forward_hook(lambda m, i, o: hook.append(1))))
+    handles[0].remove()
+    assert hook == [1] and seen == [True, False]
+    assert_close("hook", got, want)
+    with torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError,
+                                                                     match="fp32-only"):
+        step(torch.no_grad())    # refused by the general step
+    assert seen == [True, False, False]
+
+
+def test_windows_of_earlier_steps_are_kept():
+    """A cache's conv window is replaced, not written: a copy of the cache
+    dicts (with h cloned) resumes from where it was taken."""
+    hip, _ = _models()
+    idx = torch.randint(0, 203, (2, 8), generator=torch.Generator().manual_seed(2)).to(DEV)
+    cache = {}
+    with torch.no_grad():
+        hip(idx[:, :6], cache=cache)
+        hip(idx[:, 6:7], cache=cache)
+        snap = {"blocks": [dict(b, h=b["h"].clone()) for b in cache["blocks"]]}
+        first, _ = hip(idx[:, 7:8], cache=cache)
+        again, _ = hip(idx[:, 7:8], cache=snap)
+    assert torch.equal(first, again)
