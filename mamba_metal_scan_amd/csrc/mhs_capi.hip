@@ -1605,17 +1605,17 @@ namespace {
 
 // Batch rows per wave: all of a small batch, else 8 at a time (the weights'
 // rows then come from the caches again).
-template <int KIND, int RW>
+template <int KIND, int RW, int U>
 int launch_decode(const mhs::DecodeArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.rows + 4 * RW - 1) / (4 * RW))), block(256);
   if (a.batch == 1)
-    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 1, RW>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 1, RW, U>), grid, block, 0, s, a);
   else if (a.batch == 2)
-    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 2, RW>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 2, RW, U>), grid, block, 0, s, a);
   else if (a.batch <= 4)
-    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 4, RW>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 4, RW, U>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 8, RW>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((mhs::decode_product_kernel<KIND, 8, RW, 2>), grid, block, 0, s, a);
   return check_launch("decode product kernel");
 }
 
@@ -1714,12 +1714,12 @@ int mhs_decode_f32(const mhs_decode_layer* layers, int64_t n_layers, const float
     a.conv_w = p.conv_weight; a.conv_b = p.conv_bias; a.conv = p.conv;
     a.conv_sb = p.conv_sb; a.conv_sd = p.conv_sd; a.conv_sk = p.conv_sk;
     a.conv_next = p.conv_next; a.taps = (int)conv_taps;
-    rc = launch_decode<mhs::kDecIn, 2>(a, s);
+    rc = launch_decode<mhs::kDecIn, 2, 3>(a, s);
     if (rc) return rc;
     a.x = xc; a.w = p.dt_proj; a.w_b = p.B_proj; a.w_c = p.C_proj; a.K = D; a.rows = D + 2 * N;
     a.out = dt; a.out2 = bc; a.bias = p.dt_bias;
     a.dt_lo = p.dt_min; a.dt_span = p.dt_max - p.dt_min;
-    rc = launch_decode<mhs::kDecProj, 1>(a, s);
+    rc = launch_decode<mhs::kDecProj, 1, 6>(a, s);
     if (rc) return rc;
     const long long ch = batch * d_inner;
     if (N >= 4)
@@ -1733,7 +1733,7 @@ int mhs_decode_f32(const mhs_decode_layer* layers, int64_t n_layers, const float
     rc = check_launch("decode state kernel");
     if (rc) return rc;
     a.x = g; a.w = p.out_proj; a.K = D; a.rows = M; a.out = at(w.x); a.res = xin;
-    rc = launch_decode<mhs::kDecOut, 1>(a, s);
+    rc = launch_decode<mhs::kDecOut, 1, 6>(a, s);
     if (rc) return rc;
     xin = at(w.x);   // updated in place by the later blocks
   }
@@ -1741,7 +1741,7 @@ int mhs_decode_f32(const mhs_decode_layer* layers, int64_t n_layers, const float
   a.batch = nb;
   a.x = xin; a.w = head; a.K = M; a.rows = (int)vocab;
   a.norm_w = norm_weight; a.eps = eps; a.out = logits;
-  return launch_decode<mhs::kDecHead, 4>(a, s);
+  return launch_decode<mhs::kDecHead, 4, 3>(a, s);
 }
 
 }  // extern "C"

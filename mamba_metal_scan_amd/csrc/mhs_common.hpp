@@ -19,6 +19,7 @@
 namespace mhs {
 
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLn2 = 0.6931471805599453f;
 
 // v_exp_f32: 2^v, the hardware transcendental (one instruction, flushes
 // results below the fp32 normal range to zero, which the recurrence tolerates:

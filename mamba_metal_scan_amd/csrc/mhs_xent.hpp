@@ -21,7 +21,6 @@
 namespace mhs {
 
 constexpr int kXentThreads = 256;
-constexpr float kLn2 = 0.6931471805599453f;
 
 // (m, s) represents s * 2^m; combine two such partial sums. The side that
 // holds the maximum is scaled by exactly 1 (m - mm is not formed for it):

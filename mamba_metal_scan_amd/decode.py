@@ -22,49 +22,46 @@ from .linear import no_hooks
 _LAYER = struct.Struct("13Q3qQ4f")
 
 
-def _weight(mod: Optional[nn.Module], kind: type, dev: torch.device, shape: tuple
-            ) -> Optional[torch.Tensor]:
-    """mod's weight where mod is a plain module of that type without hooks and
-    the weight is fp32 of that shape, contiguous, on dev; else None."""
-    if type(mod) is not kind or not no_hooks(mod):
-        return None
-    return _param(mod._parameters.get("weight"), dev, shape)
+_f32 = torch.float32
 
 
-def _param(p: Optional[torch.Tensor], dev: torch.device, shape: tuple) -> Optional[torch.Tensor]:
-    if (p is None or p.dtype != torch.float32 or p.device != dev or p.shape != shape
-            or not p.is_contiguous()):
-        return None
-    return p
+def _plain(t: Optional[torch.Tensor], dev: torch.device, shape: tuple) -> bool:
+    """Whether t is fp32 of that shape, contiguous, on dev."""
+    return (t is not None and t.dtype is _f32 and t.shape == shape and t.device == dev
+            and t.is_contiguous())
 
 
-def _layer(block: nn.Module, bc: dict, dev: torch.device, sizes: tuple, norm_type: type,
+def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: tuple,
            conv_next: torch.Tensor) -> Optional[bytes]:
     """The block's mhs_decode_layer, or None where the native step does not
-    take it."""
-    batch, d_model, d, n, taps = sizes
+    take it: a module of another type or with hooks, a weight that is not a
+    plain fp32 parameter of its shape, a state or window that is not the
+    cache's own form."""
     m, p = block._modules, block._parameters
-    norm, conv, dt_proj = m.get("norm"), m.get("conv"), m.get("dt_proj")
-    h, win = bc.get("h"), bc.get("conv")
-    weights = (
-        _weight(norm, norm_type, dev, (d_model,)),
-        _weight(m.get("in_proj"), nn.Linear, dev, (2 * d, d_model)),
-        _weight(conv, nn.Conv1d, dev, (d, 1, taps)),
-        _param(conv._parameters.get("bias"), dev, (d,)) if conv is not None else None,
-        _weight(dt_proj, nn.Linear, dev, (d, d)),
-        _param(dt_proj._parameters.get("bias"), dev, (d,)) if dt_proj is not None else None,
-        _param(p.get("A"), dev, (d, n)),
-        _weight(m.get("B_proj"), nn.Linear, dev, (n, d)),
-        _weight(m.get("C_proj"), nn.Linear, dev, (n, d)),
-        _param(p.get("D_skip"), dev, (d,)),
-        _weight(m.get("out_proj"), nn.Linear, dev, (d_model, d)),
-        _param(h, dev, (batch, d, n)),
-    )
-    if (any(t is None for t in weights) or win is None or win.dtype != torch.float32
-            or win.device != dev or win.shape != (batch, d, taps - 1) or not norm.hip
-            or block.scan_impl == "torch" or not block.dt_min < block.dt_max
-            or any(m[k]._parameters.get("bias") is not None
-                   for k in ("in_proj", "B_proj", "C_proj", "out_proj"))):
+    try:
+        norm, in_proj, conv, dt_proj, b_proj, c_proj, out_proj = mods = (
+            m["norm"], m["in_proj"], m["conv"], m["dt_proj"], m["B_proj"], m["C_proj"],
+            m["out_proj"])
+        h, win = bc["h"], bc["conv"]
+        for mod, kind in zip(mods, kinds):
+            if (type(mod) is not kind or mod._forward_hooks or mod._forward_pre_hooks
+                    or mod._backward_hooks or mod._backward_pre_hooks):
+                return None
+        w_dt, w_conv = dt_proj._parameters, conv._parameters
+        weights = (norm._parameters["weight"], in_proj._parameters["weight"], w_conv["weight"],
+                   w_conv["bias"], w_dt["weight"], w_dt["bias"], p["A"],
+                   b_proj._parameters["weight"], c_proj._parameters["weight"], p["D_skip"],
+                   out_proj._parameters["weight"], h)
+        biases = (in_proj._parameters["bias"], b_proj._parameters["bias"],
+                  c_proj._parameters["bias"], out_proj._parameters["bias"])
+    except KeyError:
+        return None
+    for t, shape in zip(weights, shapes):
+        if not _plain(t, dev, shape):
+            return None
+    if (any(v is not None for v in biases) or win is None or win.dtype is not _f32
+            or win.shape != shapes[12] or win.device != dev or not norm.hip
+            or block.scan_impl == "torch" or not block.dt_min < block.dt_max):
         return None
     ptrs = [t.data_ptr() for t in weights]
     # The products read 16 bytes at a time.
@@ -93,19 +90,24 @@ def decode_step(model: nn.Module, x: torch.Tensor, cache: dict) -> Optional[torc
     batch, _, d_model = x.shape
     d, n, taps = first.d_inner, first.A.shape[1], first.conv.kernel_size[0]
     dev = x.device
-    head_w = _weight(head, nn.Linear, dev, (head.out_features, d_model))
-    norm_w = _weight(ln_f, type(first.norm), dev, (d_model,))
     x = x.contiguous()
-    if (head_w is None or norm_w is None or head.bias is not None or not ln_f.hip
-            or d_model % 4 or d % 4 or not 2 <= taps <= 8 or not 1 <= n <= 64
-            or batch > 65535 or (head_w.data_ptr() | norm_w.data_ptr() | x.data_ptr()) & 15):
+    if (not no_hooks(head) or not no_hooks(ln_f) or type(ln_f) is not type(first.norm)
+            or head.bias is not None or not ln_f.hip
+            or d_model % 4 or d % 4 or not 2 <= taps <= 8 or not 1 <= n <= 64 or batch > 65535):
+        return None
+    head_w, norm_w = head._parameters.get("weight"), ln_f._parameters.get("weight")
+    if (not _plain(norm_w, dev, (d_model,)) or not _plain(head_w, dev, (head.out_features, d_model))
+            or (head_w.data_ptr() | norm_w.data_ptr() | x.data_ptr()) & 15):
         return None
     windows = torch.empty((len(blocks), batch, d, taps - 1), dtype=torch.float32,
                           device=dev).unbind(0)
-    sizes = (batch, d_model, d, n, taps)
+    # In mhs_decode_layer's order; then the conv window.
+    shapes = ((d_model,), (2 * d, d_model), (d, 1, taps), (d,), (d, d), (d,), (d, n), (n, d),
+              (n, d), (d,), (d_model, d), (batch, d, n), (batch, d, taps - 1))
+    kinds = (type(ln_f), nn.Linear, nn.Conv1d, nn.Linear, nn.Linear, nn.Linear, nn.Linear)
     layers = []
     for block, bc, nxt in zip(blocks, states, windows):
-        packed = _layer(block, bc, dev, sizes, type(first.norm), nxt)
+        packed = _layer(block, bc, dev, shapes, kinds, nxt)
         if packed is None:
             return None
         layers.append(packed)

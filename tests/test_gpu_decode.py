@@ -28,6 +28,7 @@ def _models(**over):
         for b in hip.blocks:
             b.dt_proj.bias.normal_()
             b.D_skip.normal_()
+            b.A.normal_(0.0, 4.0)   # softplus on both sides of 0
             b.norm.weight.normal_(1.0, 0.1)
         hip.ln_f.weight.normal_(1.0, 0.1)
     ref = TinyMamba(MambaConfig(scan_impl="torch", **kw)).double()
