@@ -396,6 +396,14 @@ int mhs_xent_fwd_f32(const float* logits, const int64_t* targets, float* lse,
                      void* stream);
 
 /*
+ * The mean of mhs_xent_fwd_f32's loss_rows over the rows whose target is not
+ * ignore_index (mamba_metal/model.py:296-297): loss[0], NaN if there is none;
+ * n_valid[0], their count (int64). Summed in a fixed order.
+ */
+int mhs_xent_mean_f32(const float* loss_rows, const int64_t* targets, float* loss,
+                      int64_t* n_valid, int64_t rows, int64_t ignore_index, void* stream);
+
+/*
  * Its backward: dlogits[r, j] = scale[0] * (exp(logits[r, j] - lse[r]) - [j == targets[r]])
  * for rows whose target is not ignore_index, 0 for the others. scale is one
  * device float: the loss's upstream gradient over the count of rows not

@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "mhs_set_cu_count", "mhs_cu_count", "mhs_scan_fwd_noalloc_f32", "mhs_set_reduction",
     "mhs_deterministic",
     "mhs_scan_bwd_reduction", "mhs_xent_fwd_f32", "mhs_xent_bwd_f32",
+    "mhs_xent_mean_f32",
     "mhs_rmsnorm_fwd_f32", "mhs_rmsnorm_bwd_workspace_bytes", "mhs_rmsnorm_bwd_f32",
     "mhs_add_rmsnorm_fwd_f32", "mhs_gemm_preferred",
     "mhs_gemm_workspace_bytes", "mhs_gemm_f32", "mhs_decode_workspace_bytes",
@@ -135,6 +136,8 @@ def library() -> ctypes.CDLL:
             lib.mhs_scan_gated_bwd_bf16.argtypes = lib.mhs_scan_gated_bwd_f32.argtypes
             lib.mhs_xent_fwd_f32.restype = ctypes.c_int
             lib.mhs_xent_fwd_f32.argtypes = [_P] * 4 + [_I64] * 3 + [_P]
+            lib.mhs_xent_mean_f32.restype = ctypes.c_int
+            lib.mhs_xent_mean_f32.argtypes = [_P] * 4 + [_I64] * 2 + [_P]
             lib.mhs_xent_bwd_f32.restype = ctypes.c_int
             lib.mhs_xent_bwd_f32.argtypes = [_P] * 5 + [_I64] * 3 + [_P]
             lib.mhs_rmsnorm_fwd_f32.restype = ctypes.c_int
@@ -918,6 +921,38 @@ xent_fwd = _register("xent_fwd", _xent_fwd_impl, (),
 @xent_fwd.register_fake
 def _xent_fwd_fake(logits, targets, ignore_index):
     return logits.new_empty((logits.shape[0],)), logits.new_empty((logits.shape[0],))
+
+
+def _xent_mean_impl(loss_rows: torch.Tensor, targets: torch.Tensor, ignore_index: int
+                    ) -> tuple[torch.Tensor, torch.Tensor]:
+    """(loss (), n_valid ()): the mean of loss_rows over the rows whose target
+    is not ignore_index, and their count (int64)."""
+    loss = loss_rows.new_empty(())
+    n_valid = targets.new_empty(())
+    with _on(loss_rows.device):
+        rc = library().mhs_xent_mean_f32(_ptr(loss_rows), _ptr(targets), _ptr(loss),
+                                         _ptr(n_valid), targets.shape[0], ignore_index,
+                                         _stream(loss_rows.device))
+    _check(rc, "mhs_xent_mean_f32")
+    return loss, n_valid
+
+
+def _check_xent_mean(loss_rows, targets, ignore_index) -> None:
+    what = "xent_mean"
+    _on_one_device(what, loss_rows, targets)
+    _need(targets.dim() == 1 and targets.dtype == torch.int64, what,
+          f"targets must be int64 (R,); got {targets.dtype} {tuple(targets.shape)}")
+    _fp32(what, loss_rows=loss_rows)
+    _shaped(what, "loss_rows", loss_rows, targets.shape)
+    _dense(what, loss_rows=loss_rows, targets=targets)
+
+
+xent_mean = _register("xent_mean", _xent_mean_impl, (), _check_xent_mean)
+
+
+@xent_mean.register_fake
+def _xent_mean_fake(loss_rows, targets, ignore_index):
+    return loss_rows.new_empty(()), targets.new_empty(())
 
 
 def _xent_bwd_impl(logits: torch.Tensor, targets: torch.Tensor, lse: torch.Tensor,

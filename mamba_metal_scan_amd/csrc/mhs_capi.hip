@@ -1277,15 +1277,24 @@ int mhs_xent_fwd_f32(const float* logits, const int64_t* targets, float* lse, fl
   if (rows == 0) return MHS_OK;
   if (!lse || !loss_rows) return fail(MHS_EINVAL, "null pointer argument");
   const auto* t = reinterpret_cast<const long long*>(targets);
-  const bool vec = vocab % 4 == 0 && aligned16(logits);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (vec)
-    hipLaunchKernelGGL(mhs::xent_fwd_kernel<4>, dim3((unsigned)rows), dim3(mhs::kXentThreads), 0,
-                       s, logits, t, lse, loss_rows, (long long)vocab, (long long)ignore_index);
-  else
-    hipLaunchKernelGGL(mhs::xent_fwd_kernel<1>, dim3((unsigned)rows), dim3(mhs::kXentThreads), 0,
-                       s, logits, t, lse, loss_rows, (long long)vocab, (long long)ignore_index);
+  hipLaunchKernelGGL(mhs::xent_fwd_kernel<>, dim3((unsigned)rows), dim3(mhs::kXentThreads), 0, s,
+                     logits, t, lse, loss_rows, (long long)vocab, (long long)ignore_index);
   return check_launch("cross-entropy forward kernel");
+}
+
+int mhs_xent_mean_f32(const float* loss_rows, const int64_t* targets, float* loss,
+                      int64_t* n_valid, int64_t rows, int64_t ignore_index, void* stream) {
+  g_err[0] = '\0';
+  int rc = check_xent(loss_rows, targets, rows, 1);
+  if (rc) return rc;
+  if (!loss || !n_valid) return fail(MHS_EINVAL, "null pointer argument");
+  hipLaunchKernelGGL(mhs::xent_mean_kernel<>, dim3(1), dim3(mhs::kXentMeanThreads), 0,
+                     static_cast<hipStream_t>(stream), loss_rows,
+                     reinterpret_cast<const long long*>(targets), loss,
+                     reinterpret_cast<long long*>(n_valid), (long long)rows,
+                     (long long)ignore_index);
+  return check_launch("cross-entropy mean kernel");
 }
 
 int mhs_xent_bwd_f32(const float* logits, const int64_t* targets, const float* lse,
@@ -1298,16 +1307,13 @@ int mhs_xent_bwd_f32(const float* logits, const int64_t* targets, const float* l
   if (!lse || !scale || !dlogits) return fail(MHS_EINVAL, "null pointer argument");
   if (dlogits == logits) return fail(MHS_EINVAL, "dlogits may not alias logits");
   const auto* t = reinterpret_cast<const long long*>(targets);
-  const bool vec = vocab % 4 == 0 && aligned16(logits) && aligned16(dlogits);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (vec)
-    hipLaunchKernelGGL(mhs::xent_bwd_kernel<4>, dim3((unsigned)rows), dim3(mhs::kXentThreads), 0,
-                       s, logits, t, lse, scale, dlogits, (long long)vocab,
-                       (long long)ignore_index);
-  else
-    hipLaunchKernelGGL(mhs::xent_bwd_kernel<1>, dim3((unsigned)rows), dim3(mhs::kXentThreads), 0,
-                       s, logits, t, lse, scale, dlogits, (long long)vocab,
-                       (long long)ignore_index);
+  // The rows of both start at the same place modulo 16 bytes.
+  const bool same = ((reinterpret_cast<uintptr_t>(logits) ^ reinterpret_cast<uintptr_t>(dlogits)) &
+                     15u) == 0;
+  hipLaunchKernelGGL((same ? &mhs::xent_bwd_kernel<true> : &mhs::xent_bwd_kernel<false>),
+                     dim3((unsigned)rows), dim3(mhs::kXentThreads), 0,
+                     static_cast<hipStream_t>(stream), logits, t, lse, scale, dlogits,
+                     (long long)vocab, (long long)ignore_index);
   return check_launch("cross-entropy backward kernel");
 }
 

@@ -62,54 +62,66 @@ __device__ __forceinline__ void block_lse2(float& m, float& s) {
   for (int w = 1; w < kXentThreads / 64; ++w) lse2_combine(m, s, red[0][w], red[1][w]);
 }
 
-// VEC: 4 (vocab a multiple of 4, rows 16-byte aligned: float4 loads) or 1.
+// A row of any length at any 4-byte alignment: up to 3 elements to the first
+// 16-byte boundary (head), whole float4s (n4), up to 3 more (tail; with the
+// head at most 6 single elements, `ends`, one per thread).
+struct XentRow {
+  int head, ends;
+  long long n4;
+  __device__ __forceinline__ XentRow(const float* x, long long vocab) {
+    head = (int)min((long long)((16u - ((unsigned)reinterpret_cast<uintptr_t>(x) & 15u)) & 15u) / 4,
+                    vocab);
+    n4 = (vocab - head) / 4;
+    ends = (int)(vocab - 4 * n4);
+  }
+  // The index of single element j < ends.
+  __device__ __forceinline__ long long end(int j) const { return j < head ? j : 4 * n4 + j; }
+};
+
+// HBM-bound: each logit read once, in 16-byte loads also where the vocabulary
+// is no multiple of 4 (4096 x 50257: 274 us with 4-byte loads, 180 so, 4.6
+// TB/s).
 // A target outside [0, vocab) that is not ignore_index gives loss NaN (the
 // framework raises a device-side assertion there).
-template <int VEC>
+template <int UNUSED = 0>
 __global__ void __launch_bounds__(kXentThreads)
 xent_fwd_kernel(const float* __restrict__ logits, const long long* __restrict__ targets,
                 float* __restrict__ lse, float* __restrict__ loss_rows, long long vocab,
                 long long ignore_index) {
   const long long r = blockIdx.x;
   const float* x = logits + r * vocab;
+  const XentRow row(x, vocab);
   float m = -INFINITY, s = 0.f;
-  if constexpr (VEC == 4) {
-    const float4* x4 = reinterpret_cast<const float4*>(x);
-    const long long n4 = vocab / 4;
-    constexpr int U = 4;   // float4 loads per update of the running maximum
-    long long i = threadIdx.x;
-    for (; i + (U - 1) * kXentThreads < n4; i += U * kXentThreads) {
-      float y[4 * U];
+  if ((int)threadIdx.x < row.ends) lse2_combine(m, s, x[row.end(threadIdx.x)] * kLog2e, 1.f);
+  const float4* x4 = reinterpret_cast<const float4*>(x + row.head);
+  constexpr int U = 4;   // float4 loads per update of the running maximum
+  long long i = threadIdx.x;
+  for (; i + (U - 1) * kXentThreads < row.n4; i += U * kXentThreads) {
+    float y[4 * U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float4 v = x4[i + u * kXentThreads];
-        y[4 * u] = v.x * kLog2e;
-        y[4 * u + 1] = v.y * kLog2e;
-        y[4 * u + 2] = v.z * kLog2e;
-        y[4 * u + 3] = v.w * kLog2e;
-      }
-      float mc = y[0];
+    for (int u = 0; u < U; ++u) {
+      const float4 v = x4[i + u * kXentThreads];
+      y[4 * u] = v.x * kLog2e;
+      y[4 * u + 1] = v.y * kLog2e;
+      y[4 * u + 2] = v.z * kLog2e;
+      y[4 * u + 3] = v.w * kLog2e;
+    }
+    float mc = y[0];
 #pragma unroll
-      for (int k = 1; k < 4 * U; ++k) mc = fmaxf(mc, y[k]);
-      const float sh = lse2_shift(mc);
-      float sc = 0.f;
+    for (int k = 1; k < 4 * U; ++k) mc = fmaxf(mc, y[k]);
+    const float sh = lse2_shift(mc);
+    float sc = 0.f;
 #pragma unroll
-      for (int k = 0; k < 4 * U; ++k) sc += exp2_hw(y[k] - sh);
-      lse2_combine(m, s, mc, sc);
-    }
-    for (; i < n4; i += kXentThreads) {
-      const float4 v = x4[i];
-      const float y0 = v.x * kLog2e, y1 = v.y * kLog2e, y2 = v.z * kLog2e, y3 = v.w * kLog2e;
-      const float mc = fmaxf(fmaxf(y0, y1), fmaxf(y2, y3));
-      const float sh = lse2_shift(mc);
-      lse2_combine(m, s, mc,
-                   exp2_hw(y0 - sh) + exp2_hw(y1 - sh) + exp2_hw(y2 - sh) + exp2_hw(y3 - sh));
-    }
-  } else {
-    for (long long j = threadIdx.x; j < vocab; j += kXentThreads) {
-      const float y = x[j] * kLog2e;
-      lse2_combine(m, s, y, 1.f);
-    }
+    for (int k = 0; k < 4 * U; ++k) sc += exp2_hw(y[k] - sh);
+    lse2_combine(m, s, mc, sc);
+  }
+  for (; i < row.n4; i += kXentThreads) {
+    const float4 v = x4[i];
+    const float y0 = v.x * kLog2e, y1 = v.y * kLog2e, y2 = v.z * kLog2e, y3 = v.w * kLog2e;
+    const float mc = fmaxf(fmaxf(y0, y1), fmaxf(y2, y3));
+    const float sh = lse2_shift(mc);
+    lse2_combine(m, s, mc,
+                 exp2_hw(y0 - sh) + exp2_hw(y1 - sh) + exp2_hw(y2 - sh) + exp2_hw(y3 - sh));
   }
   block_lse2(m, s);
   if (threadIdx.x == 0) {
@@ -122,7 +134,42 @@ xent_fwd_kernel(const float* __restrict__ logits, const long long* __restrict__ 
   }
 }
 
-template <int VEC>
+// loss[0] = the sum of loss_rows over the count of targets that are not
+// ignore_index (0 / 0 = NaN, as the framework's mean); n_valid[0] = the count.
+// One block, in a fixed order: a launch where the framework takes four.
+constexpr int kXentMeanThreads = 1024;
+template <int UNUSED = 0>
+__global__ void __launch_bounds__(kXentMeanThreads)
+xent_mean_kernel(const float* __restrict__ loss_rows, const long long* __restrict__ targets,
+                 float* __restrict__ loss, long long* __restrict__ n_valid, long long rows,
+                 long long ignore_index) {
+  __shared__ double sums[kXentMeanThreads];
+  __shared__ int counts[kXentMeanThreads];   // rows < 2^31
+  double s = 0.0;
+  int n = 0;
+  for (long long r = threadIdx.x; r < rows; r += kXentMeanThreads) {
+    s += loss_rows[r];
+    n += targets[r] != ignore_index;
+  }
+  sums[threadIdx.x] = s;
+  counts[threadIdx.x] = n;
+  for (int h = kXentMeanThreads / 2; h >= 1; h >>= 1) {
+    __syncthreads();
+    if ((int)threadIdx.x < h) {
+      sums[threadIdx.x] += sums[threadIdx.x + h];
+      counts[threadIdx.x] += counts[threadIdx.x + h];
+    }
+  }
+  if (threadIdx.x == 0) {
+    loss[0] = (float)(sums[0] / counts[0]);
+    n_valid[0] = counts[0];
+  }
+}
+
+// HBM-bound: each logit read and each gradient written once (4096 x 50257:
+// 370 us with 4-byte accesses, 334 so, 4.9 TB/s, the rate of a copy). SAME: dlogits has logits' alignment
+// modulo 16 bytes; otherwise its elements are stored one by one.
+template <bool SAME>
 __global__ void __launch_bounds__(kXentThreads)
 xent_bwd_kernel(const float* __restrict__ logits, const long long* __restrict__ targets,
                 const float* __restrict__ lse, const float* __restrict__ scale,
@@ -134,29 +181,36 @@ xent_bwd_kernel(const float* __restrict__ logits, const long long* __restrict__ 
   const bool ignored = t == ignore_index;
   const float g = ignored ? 0.f : scale[0];
   const float l2 = lse[r] * kLog2e;
-  if constexpr (VEC == 4) {
-    const float4* x4 = reinterpret_cast<const float4*>(x);
-    float4* d4 = reinterpret_cast<float4*>(dx);
-    const long long n4 = vocab / 4;
-    for (long long i = threadIdx.x; i < n4; i += kXentThreads) {
-      const float4 v = x4[i];
-      float4 p = make_float4(exp2_hw(__builtin_fmaf(v.x, kLog2e, -l2)),
-                             exp2_hw(__builtin_fmaf(v.y, kLog2e, -l2)),
-                             exp2_hw(__builtin_fmaf(v.z, kLog2e, -l2)),
-                             exp2_hw(__builtin_fmaf(v.w, kLog2e, -l2)));
-      if ((t >> 2) == i) {   // the target's element: p - 1 (one thread, once)
-        const int k = (int)(t & 3);
-        if (k == 0) p.x -= 1.f;
-        if (k == 1) p.y -= 1.f;
-        if (k == 2) p.z -= 1.f;
-        if (k == 3) p.w -= 1.f;
-      }
-      d4[i] = make_float4(g * p.x, g * p.y, g * p.z, g * p.w);
+  const XentRow row(x, vocab);
+  if ((int)threadIdx.x < row.ends) {
+    const long long j = row.end(threadIdx.x);
+    const float p = exp2_hw(__builtin_fmaf(x[j], kLog2e, -l2));
+    dx[j] = g * (j == t ? p - 1.f : p);
+  }
+  const float4* x4 = reinterpret_cast<const float4*>(x + row.head);
+  const long long th = t - row.head;   // the target counted from the float4s
+  for (long long i = threadIdx.x; i < row.n4; i += kXentThreads) {
+    const float4 v = x4[i];
+    float4 p = make_float4(exp2_hw(__builtin_fmaf(v.x, kLog2e, -l2)),
+                           exp2_hw(__builtin_fmaf(v.y, kLog2e, -l2)),
+                           exp2_hw(__builtin_fmaf(v.z, kLog2e, -l2)),
+                           exp2_hw(__builtin_fmaf(v.w, kLog2e, -l2)));
+    if ((th >> 2) == i) {   // the target's element: p - 1 (one thread, once)
+      const int k = (int)(th & 3);
+      if (k == 0) p.x -= 1.f;
+      if (k == 1) p.y -= 1.f;
+      if (k == 2) p.z -= 1.f;
+      if (k == 3) p.w -= 1.f;
     }
-  } else {
-    for (long long j = threadIdx.x; j < vocab; j += kXentThreads) {
-      const float p = exp2_hw(__builtin_fmaf(x[j], kLog2e, -l2));
-      dx[j] = g * (j == t ? p - 1.f : p);
+    p = make_float4(g * p.x, g * p.y, g * p.z, g * p.w);
+    if constexpr (SAME) {
+      reinterpret_cast<float4*>(dx + row.head)[i] = p;
+    } else {
+      float* d = dx + row.head + 4 * i;
+      d[0] = p.x;
+      d[1] = p.y;
+      d[2] = p.z;
+      d[3] = p.w;
     }
   }
 }

@@ -28,11 +28,11 @@ class CrossEntropyHIP(torch.autograd.Function):
         logits = logits.contiguous()
         targets = targets.contiguous()
         lse, loss_rows = _native.dispatch("xent_fwd")(logits, targets, ignore_index)
-        n_valid = (targets != ignore_index).sum()
+        # 0 / 0 = NaN when every row is ignored, as the framework's mean.
+        loss, n_valid = _native.dispatch("xent_mean")(loss_rows, targets, ignore_index)
         ctx.save_for_backward(logits, targets, lse, n_valid)
         ctx.ignore_index = ignore_index
-        # 0 / 0 = NaN when every row is ignored, as the framework's mean.
-        return loss_rows.sum() / n_valid
+        return loss
 
     @staticmethod
     def backward(ctx, g):

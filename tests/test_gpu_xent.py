@@ -164,3 +164,33 @@ def test_op_argument_errors():
     lse = torch.zeros(4, device=DEV)
     with pytest.raises(HipScanError, match="scale"):
         torch.ops.mamba_hip.xent_bwd(logits, targets, lse, torch.ones(2, device=DEV), -100)
+
+
+@pytest.mark.parametrize("vocab", [2, 3, 5, 7, 1023, 1025, 4099])
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+def test_rows_of_any_length_and_alignment(vocab, offset):
+    """Row starts at every alignment modulo 16 bytes, the gradient's rows
+    aligned with the logits' (offset 0) or not, targets at both ends."""
+    rows = 6
+    logits, targets = _case(rows, vocab, seed=vocab, ignore_frac=0.0)
+    targets[:4] = torch.tensor([0, min(3, vocab - 1), vocab - 1, max(0, vocab - 4)])
+    buf = torch.empty(rows * vocab + offset, device=DEV)
+    view = buf[offset:].view(rows, vocab)
+    view.copy_(logits.to(DEV))
+    l_ref, g_ref = _reference(logits, targets, 1.5)
+    l_hip, g_hip = _hip(logits, targets, 1.5, storage=view)
+    assert _rel(l_hip, l_ref) <= 1e-5 and _rel(g_hip, g_ref) <= 1e-5
+
+
+@pytest.mark.parametrize("rows", [1, 1023, 1024, 1025, 5000])
+def test_mean_over_rows(rows):
+    """xent_mean on both sides of its block's 1024 rows."""
+    g = torch.Generator().manual_seed(rows)
+    loss_rows = torch.rand(rows, generator=g)
+    targets = torch.randint(0, 9, (rows,), generator=g)
+    targets[1::7] = -100
+    loss_rows[1::7] = 0.0
+    loss, n = torch.ops.mamba_hip.xent_mean(loss_rows.to(DEV), targets.to(DEV), -100)
+    valid = (targets != -100).sum()
+    assert n.item() == valid.item()
+    assert abs(loss.item() - loss_rows.double().sum().item() / valid.item()) <= 1e-6
