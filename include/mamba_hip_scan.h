@@ -516,6 +516,54 @@ int mhs_decode_f32(const mhs_decode_layer* layers, int64_t n_layers, const float
                    int64_t conv_taps, int64_t vocab, void* workspace, size_t workspace_bytes,
                    void* stream);
 
+/*
+ * A whole MambaBlock, fp32, as one call per direction (the reference's
+ * MambaBlock.forward over a sequence, mamba_metal/model.py:225-256): the
+ * residual stream's update x_out = x + delta by the previous block's output
+ * (delta NULL: x itself, x_out unused), the RMSNorm, in_proj, the conv with
+ * SiLU, the merged dt / B / C projection, the gated scan, the output gate and
+ * out_proj; out receives the block's output before its own residual add.
+ * d_model (up to 2048), d_inner and d_state are multiples of 4; the weights
+ * are contiguous and 16-byte aligned, as nn.Linear / nn.Conv1d hold them.
+ * x, delta, x_out, out: (batch, seqlen, d_model); xz: (batch, seqlen,
+ * 2 d_inner), in_proj's output, kept for the backward (its first half holds the
+ * conv window of a recurrent cache); saved: mhs_block_saved_bytes bytes, what
+ * else the backward needs, fully written (with_ckpt 0: no checkpoints, no
+ * backward); h_last: NULL or (batch, d_inner, d_state), the final state.
+ * The backward takes the forward's x (x_out where there was a delta), xz,
+ * saved, the gradients of out (dout) and, or NULL, of x_out (dres); x's and
+ * delta's gradient are both g->x. g->proj is the merged projection's weight
+ * gradient, rows [dt | B | C]; g->in_proj and g->out_proj may be NULL. Its
+ * workspace depends on the reduction mode (mhs_set_reduction) at the query.
+ * Workspaces and saved are 256-byte aligned.
+ */
+typedef struct mhs_block_weights {
+  const float *norm_weight, *in_proj, *conv_weight, *conv_bias, *dt_proj, *dt_bias, *A, *B_proj,
+      *C_proj, *D_skip, *out_proj;
+  float eps, dt_min, dt_max, unused;
+} mhs_block_weights;
+typedef struct mhs_block_grads {
+  float *x, *norm_weight, *in_proj, *conv_weight, *conv_bias, *proj, *dt_bias, *A, *D_skip,
+      *out_proj;
+} mhs_block_grads;
+size_t mhs_block_saved_bytes(int64_t batch, int64_t seqlen, int64_t d_model, int64_t d_inner,
+                             int64_t d_state, int64_t conv_taps, int64_t chunk, int with_ckpt);
+size_t mhs_block_fwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t d_model,
+                                     int64_t d_inner, int64_t d_state, int64_t conv_taps);
+int mhs_block_fwd_f32(const mhs_block_weights* w, const float* x, const float* delta, float* x_out,
+                      float* out, float* xz, void* saved, float* h_last, int64_t batch,
+                      int64_t seqlen, int64_t d_model, int64_t d_inner, int64_t d_state,
+                      int64_t conv_taps, int64_t chunk, int with_ckpt, void* workspace,
+                      size_t workspace_bytes, void* stream);
+size_t mhs_block_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t d_model,
+                                     int64_t d_inner, int64_t d_state, int64_t conv_taps,
+                                     int64_t chunk);
+int mhs_block_bwd_f32(const mhs_block_weights* w, const float* x, const float* xz,
+                      const void* saved, const float* dout, const float* dres,
+                      const mhs_block_grads* g, int64_t batch, int64_t seqlen, int64_t d_model,
+                      int64_t d_inner, int64_t d_state, int64_t conv_taps, int64_t chunk,
+                      void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

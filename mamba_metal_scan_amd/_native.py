@@ -39,7 +39,8 @@ EXPORTED_SYMBOLS = (
     "mhs_rmsnorm_fwd_f32", "mhs_rmsnorm_bwd_workspace_bytes", "mhs_rmsnorm_bwd_f32",
     "mhs_add_rmsnorm_fwd_f32", "mhs_gemm_preferred",
     "mhs_gemm_workspace_bytes", "mhs_gemm_f32", "mhs_decode_workspace_bytes",
-    "mhs_decode_f32",
+    "mhs_decode_f32", "mhs_block_saved_bytes", "mhs_block_fwd_workspace_bytes",
+    "mhs_block_fwd_f32", "mhs_block_bwd_workspace_bytes", "mhs_block_bwd_f32",
 )
 
 # Size of the static device scratch of mhs_scan_fwd_noalloc_f32 (the header's
@@ -160,6 +161,18 @@ def library() -> ctypes.CDLL:
             lib.mhs_decode_f32.restype = ctypes.c_int
             lib.mhs_decode_f32.argtypes = ([ctypes.c_char_p, _I64, _P, _P, _F32, _P, _P]
                                            + [_I64] * 6 + [_P, ctypes.c_size_t, _P])
+            lib.mhs_block_saved_bytes.restype = ctypes.c_size_t
+            lib.mhs_block_saved_bytes.argtypes = [_I64] * 7 + [ctypes.c_int]
+            lib.mhs_block_fwd_workspace_bytes.restype = ctypes.c_size_t
+            lib.mhs_block_fwd_workspace_bytes.argtypes = [_I64] * 6
+            lib.mhs_block_bwd_workspace_bytes.restype = ctypes.c_size_t
+            lib.mhs_block_bwd_workspace_bytes.argtypes = [_I64] * 7
+            lib.mhs_block_fwd_f32.restype = ctypes.c_int
+            lib.mhs_block_fwd_f32.argtypes = ([ctypes.c_char_p] + [_P] * 7 + [_I64] * 7
+                                              + [ctypes.c_int, _P, ctypes.c_size_t, _P])
+            lib.mhs_block_bwd_f32.restype = ctypes.c_int
+            lib.mhs_block_bwd_f32.argtypes = ([ctypes.c_char_p] + [_P] * 5 + [ctypes.c_char_p]
+                                              + [_I64] * 7 + [_P, ctypes.c_size_t, _P])
             _lib = lib
     return _lib
 
@@ -188,8 +201,11 @@ def _stream(dev: torch.device) -> int:
 def _on(dev: torch.device):
     """torch.cuda.device(dev), or no context switch when dev is already current."""
     if dev.index is None or dev.index == torch.cuda.current_device():
-        return contextlib.nullcontext()
+        return _NO_SWITCH
     return torch.cuda.device(dev)
+
+
+_NO_SWITCH = contextlib.nullcontext()
 
 
 def num_chunks(seqlen: int, chunk: int) -> int:
@@ -246,24 +262,26 @@ def bwd_reduction(batch: int, seqlen: int, d_inner: int, d_state: int, chunk: in
     return mode
 
 
-@contextlib.contextmanager
-def _bwd_reduction():
+class _bwd_reduction:
     """Around one backward call (workspace query and launch): the fixed-order
     reduction while torch's deterministic algorithms are enabled, else the
     process-wide mode. Every backward holds the lock from its workspace query
     to its launch, so that a deterministic call in another thread cannot
     switch the library's mode in between (the workspace would then be sized
     for the other reduction)."""
-    with _reduction_lock:
-        if not torch.are_deterministic_algorithms_enabled():
-            yield
-            return
-        lib = library()
-        lib.mhs_set_reduction(REDUCTION_FIXED)
+
+    def __enter__(self):
+        _reduction_lock.acquire()
+        self.fixed = torch.are_deterministic_algorithms_enabled()
+        if self.fixed:
+            library().mhs_set_reduction(REDUCTION_FIXED)
+
+    def __exit__(self, *exc):
         try:
-            yield
+            if self.fixed:
+                library().mhs_set_reduction(_reduction)
         finally:
-            lib.mhs_set_reduction(_reduction)
+            _reduction_lock.release()
 
 
 def set_cu_count(cus: int) -> None:
@@ -411,22 +429,33 @@ def dispatch(name: str):
     return _IMPLS[name]
 
 
+def scan_fwd_into(x, dt, aneg, b_in, c_in, chunk: int, with_ckpt: bool, want_state: bool):
+    """(y, ckpt or None, h_last or None): the forward without the outputs that
+    are not asked for."""
+    bt, t_len, d = x.shape
+    n = aneg.shape[1]
+    dev = x.device
+    y = torch.empty_like(x)
+    ckpt = aneg.new_empty((bt, num_chunks(t_len, chunk), d, n)) if with_ckpt else None
+    h_last = aneg.new_empty((bt, d, n)) if want_state else None
+    lib = library()
+    nbytes = lib.mhs_scan_fwd_workspace_bytes(bt, t_len, d, n)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    fn = lib.mhs_scan_fwd_bf16 if x.dtype is torch.bfloat16 else lib.mhs_scan_fwd_ws_f32
+    with _on(dev):
+        rc = fn(x.data_ptr(), dt.data_ptr(), aneg.data_ptr(), b_in.data_ptr(), c_in.data_ptr(),
+                y.data_ptr(), _ptr(ckpt), _ptr(h_last), _ptr(ws), nbytes, bt, t_len, d, n, chunk,
+                _stream(dev))
+    _check(rc, "scan forward")
+    return y, ckpt, h_last
+
+
 def _scan_fwd_impl(x: torch.Tensor, dt: torch.Tensor, aneg: torch.Tensor, b_in: torch.Tensor,
              c_in: torch.Tensor, chunk: int, with_ckpt: bool
              ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """y (B,T,D), ckpt (B,ceil(T/chunk),D,N) or an empty tensor, h_last (B,D,N)."""
-    bt, t_len, d = x.shape
-    n = aneg.shape[1]
-    y, ckpt, h_last = _fwd_outputs(x, n, chunk, with_ckpt)
-    ws, ws_bytes = _fwd_workspace(x, n)
-    lib = library()
-    fn = lib.mhs_scan_fwd_bf16 if x.dtype == torch.bfloat16 else lib.mhs_scan_fwd_ws_f32
-    with _on(x.device):
-        rc = fn(_ptr(x), _ptr(dt), _ptr(aneg), _ptr(b_in), _ptr(c_in), _ptr(y),
-                _ptr(ckpt) if with_ckpt else None, _ptr(h_last), _ptr(ws), ws_bytes,
-                bt, t_len, d, n, chunk, _stream(x.device))
-    _check(rc, "scan forward")
-    return y, ckpt, h_last
+    y, ckpt, h_last = scan_fwd_into(x, dt, aneg, b_in, c_in, chunk, with_ckpt, True)
+    return y, aneg.new_empty((0,)) if ckpt is None else ckpt, h_last
 
 
 scan_fwd = _register(
@@ -448,17 +477,19 @@ def _scan_bwd_impl(x: torch.Tensor, dt: torch.Tensor, aneg: torch.Tensor, b_in: 
     bt, t_len, d = x.shape
     n = aneg.shape[1]
     lib = library()
+    dev = x.device
     dx = torch.empty_like(x)
     ddt = torch.empty_like(dt)
     daneg = torch.empty_like(aneg)
     db = torch.empty_like(b_in)
     dc = torch.empty_like(c_in)
-    fn = lib.mhs_scan_bwd_bf16 if x.dtype == torch.bfloat16 else lib.mhs_scan_bwd_f32
-    with _bwd_reduction(), _on(x.device):
+    fn = lib.mhs_scan_bwd_bf16 if x.dtype is torch.bfloat16 else lib.mhs_scan_bwd_f32
+    with _bwd_reduction(), _on(dev):
         ws, ws_bytes = _bwd_workspace(x, n, chunk)
-        rc = fn(_ptr(x), _ptr(dt), _ptr(aneg), _ptr(b_in), _ptr(c_in), _ptr(dy),
-                _ptr(dh_last), _ptr(ckpt), _ptr(dx), _ptr(ddt), _ptr(daneg), _ptr(db), _ptr(dc),
-                _ptr(ws), ws_bytes, bt, t_len, d, n, chunk, _stream(x.device))
+        rc = fn(x.data_ptr(), dt.data_ptr(), aneg.data_ptr(), b_in.data_ptr(), c_in.data_ptr(),
+                dy.data_ptr(), _ptr(dh_last), ckpt.data_ptr(), dx.data_ptr(), ddt.data_ptr(),
+                daneg.data_ptr(), db.data_ptr(), dc.data_ptr(), ws.data_ptr(), ws_bytes, bt,
+                t_len, d, n, chunk, _stream(dev))
     _check(rc, "scan backward")
     return dx, ddt, daneg, db, dc
 

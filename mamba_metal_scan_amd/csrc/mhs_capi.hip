@@ -1467,43 +1467,46 @@ int mhs_rmsnorm_bwd_f32(const float* dy, const float* x, const float* weight, co
 
 namespace {
 
-// Split-K of a product of tiles 128 x 128 tiles and kt k tiles (16 deep) on
-// `cus` CUs, three blocks each: the blocks come in rounds of cus (the blocks
-// of a CU share its matrix cores, so the last round's idle CUs are what is
-// lost), a block's first loads and epilogue cost about 4 k tiles, and the
-// partials are written and read back once. A k tile of a tile takes 0.6 us
-// of a CU (measured at 144, 320 and 768 tiles with 1-8 splits: the least of
-// this estimate was within 6% of the fastest). A split sums at most
-// kGemmMaxChain k's in one chain of MFMA additions, so that the result's error
-// stays below that of a plain fp32 product (relative 2-norm against 64 bits at
-// K 1432, 8192: 5.8e-7, 1.44e-6; rocBLAS 6.4e-7, 1.62e-6; at 32768 in one
-// chain 3.0e-6 against 2.0e-6).
+// Tile and split-K of a product on `cus` CUs. The blocks come in rounds of
+// cus; a k tile (16 deep) of a 128 x 128 tile takes 0.6 us of a CU (the three
+// blocks of a CU share its matrix cores), of a 64 x 64 tile 0.25 us and at
+// least 0.45 us alone; a block's first loads and epilogue cost about 4 k
+// tiles; the partials of a split are written and read back once. Measured at
+// 144, 320 and 768 large tiles with 1-8 splits and at 64 to 864 small ones:
+// the least of this estimate was within 6% of the fastest. (512 x 1712 x 384:
+// 17 us small, 22 large; 2048 x 1712 x 384: 30 and 29.)
+// A split sums at most kGemmMaxChain k's in one chain of MFMA additions, so
+// that the result's error stays below that of a plain fp32 product (relative
+// 2-norm against 64 bits at K 1432, 8192: 5.8e-7, 1.44e-6; rocBLAS 6.4e-7,
+// 1.62e-6; at 32768 in one chain 3.0e-6 against 2.0e-6).
 constexpr int kGemmMaxChain = 4096;
 constexpr int kGemmMaxSplits = 32;
 
 struct GemmPlan {
-  int grid_m = 0, grid_n = 0, splits = 1, kt_per_split = 0;
+  int tile = 0, grid_m = 0, grid_n = 0, splits = 1, kt_per_split = 0;
 };
 
 GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
   GemmPlan p;
-  p.grid_m = (int)((M + mhs::kGemmBM - 1) / mhs::kGemmBM);
-  p.grid_n = (int)((N + mhs::kGemmBN - 1) / mhs::kGemmBN);
   const int cus = device_cus();
-  const double tiles = (double)p.grid_m * p.grid_n;
   const int kt = (int)((K + mhs::kGemmBK - 1) / mhs::kGemmBK);
   const int least = (int)((K + kGemmMaxChain - 1) / kGemmMaxChain);
-  // The reduction reads whole float4s: other widths are not split further
-  // than the chain's length needs.
+  // The reduction reads whole float4s: other widths are not split.
   const int most = N % 4 == 0 ? std::max(least, std::min(kGemmMaxSplits, kt / 8)) : 1;
   double best = 0;
-  for (int s = std::min(least, most); s <= most; ++s) {
-    const double blocks = tiles * s, rounds = std::ceil(blocks / cus);
-    const double us = rounds * (kt / (double)s + 4) * 0.6 +
-                      (s > 1 ? (2 * s + 1) * (double)M * N * 4 / 4.8e6 + 4 : 0);
-    if (p.kt_per_split == 0 || us < best) {
+  for (const int tile : {mhs::kGemmTile, mhs::kGemmSmallTile}) {
+    const int64_t gm = (M + tile - 1) / tile, gn = (N + tile - 1) / tile;
+    if (gm * gn > 0x7FFFFFFF) continue;
+    const double per_kt = tile == mhs::kGemmTile ? 0.6 : 0.25, alone = std::max(per_kt, 0.45);
+    for (int s = std::min(least, most); s <= most; ++s) {
+      const double rounds = std::ceil((double)gm * gn * s / cus);
+      const double us = std::max(rounds * per_kt, alone) * (kt / (double)s + 4) +
+                        (s > 1 ? (2 * s + 1) * (double)M * N * 4 / 4.8e6 + 4 : 0);
+      if (p.kt_per_split != 0 && us >= best) continue;
       best = us;
-      p.splits = s;
+      p.tile = tile;
+      p.grid_m = (int)gm;
+      p.grid_n = (int)gn;
       p.kt_per_split = (kt + s - 1) / s;
     }
   }
@@ -1519,7 +1522,7 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
 bool gemm_preferred(int64_t M, int64_t N, int64_t K) {
   const GemmPlan p = gemm_plan(M, N, K);
   return (double)M * N * K >= 1073741824.0 &&
-         (double)M * N >= 0.7 * (double)p.grid_m * p.grid_n * mhs::kGemmBM * mhs::kGemmBN;
+         (double)M * N >= 0.7 * (double)p.grid_m * p.grid_n * p.tile * p.tile;
 }
 
 int check_gemm(int64_t M, int64_t N, int64_t K) {
@@ -1588,12 +1591,15 @@ int mhs_gemm_f32(int form, const float* a, int64_t lda, const float* b, int64_t 
     g.ldc = n;
     g.accumulate = 0;
   }
-  const auto fn = form == MHS_GEMM_NT ? &mhs::gemm3_kernel<true, true>
-                  : form == MHS_GEMM_NN ? &mhs::gemm3_kernel<true, false>
-                                        : &mhs::gemm3_kernel<false, false>;
+  const bool large = p.tile == mhs::kGemmTile;
+  constexpr int L = mhs::kGemmTile, S = mhs::kGemmSmallTile;
+  const auto fn =
+      form == MHS_GEMM_NT ? (large ? &mhs::gemm3_kernel<true, true, L> : &mhs::gemm3_kernel<true, true, S>)
+      : form == MHS_GEMM_NN
+          ? (large ? &mhs::gemm3_kernel<true, false, L> : &mhs::gemm3_kernel<true, false, S>)
+          : (large ? &mhs::gemm3_kernel<false, false, L> : &mhs::gemm3_kernel<false, false, S>);
   hipLaunchKernelGGL(fn, dim3((unsigned)p.grid_m * (unsigned)p.grid_n, (unsigned)p.splits),
-                     dim3(mhs::kGemmThreads), mhs::gemm_lds_bytes(mhs::kGemmBM, mhs::kGemmBN), s,
-                     g);
+                     dim3(mhs::kGemmThreads), mhs::gemm_lds_bytes(p.tile, p.tile), s, g);
   rc = check_launch("matrix product kernel");
   if (rc || p.splits == 1) return rc;
   const long long n4 = (long long)m * (n / 4);
@@ -1748,6 +1754,258 @@ int mhs_decode_f32(const mhs_decode_layer* layers, int64_t n_layers, const float
   a.x = xin; a.w = head; a.K = M; a.rows = (int)vocab;
   a.norm_w = norm_weight; a.eps = eps; a.out = logits;
   return launch_decode<mhs::kDecHead, 4, 3>(a, s);
+}
+
+}  // extern "C"
+
+// ------------------------------------------------------------ a whole block
+
+namespace {
+
+// What a block's forward leaves for its backward, in one buffer: the norm's
+// output and 1 / rms, the conv's output, the projections [dt | B | C], the
+// scan's y, the gated y, the merged projection weight, the checkpoints.
+struct BlockSaved {
+  size_t h, rstd, xc, proj, y, gate, wproj, ckpt, total;
+};
+
+struct BlockDims {
+  int64_t B, T, M, dm, d, N, taps, chunk, P;   // M = B T, P = d + 2 N
+};
+
+BlockSaved block_saved(const BlockDims& s, bool with_ckpt) {
+  BlockSaved o;
+  size_t off = 0;
+  auto take = [&](size_t floats) {
+    const size_t at = off;
+    off += round_up(floats * 4, 256);
+    return at;
+  };
+  o.h = take((size_t)s.M * s.dm);
+  o.rstd = take((size_t)s.M);
+  o.xc = take((size_t)s.M * s.d);
+  o.proj = take((size_t)s.M * s.P);
+  o.y = take((size_t)s.M * s.d);
+  o.gate = take((size_t)s.M * s.d);
+  o.wproj = take((size_t)s.P * s.d);
+  o.ckpt = take(with_ckpt ? (size_t)s.B * ((s.T + s.chunk - 1) / s.chunk) * s.d * s.N : 0);
+  o.total = off;
+  return o;
+}
+
+int block_dims(int64_t batch, int64_t seqlen, int64_t d_model, int64_t d_inner, int64_t d_state,
+               int64_t taps, int64_t chunk, BlockDims& s) {
+  int rc = check_shape(batch, seqlen, d_inner, d_state, chunk);
+  if (rc) return rc;
+  if (d_model < 4 || d_model > 256 * mhs::kNormMaxNV || d_model % 4 || d_inner % 4 || d_state % 4)
+    return fail(MHS_EINVAL, "d_model (up to %d), d_inner and d_state must be multiples of 4; got "
+                "%lld %lld %lld", 256 * mhs::kNormMaxNV, (long long)d_model, (long long)d_inner,
+                (long long)d_state);
+  if (taps < 1 || taps > mhs::kConvMaxK)
+    return fail(MHS_EINVAL, "kernel_size %lld unsupported (1..%d)", (long long)taps,
+                mhs::kConvMaxK);
+  if (2 * d_inner >= (1LL << 22) || batch * seqlen > (1LL << 30))
+    return fail(MHS_EINVAL, "sizes too large");
+  s = BlockDims{batch, seqlen, batch * seqlen, d_model, d_inner, d_state, taps, chunk,
+                d_inner + 2 * d_state};
+  return MHS_OK;
+}
+
+size_t gemm_ws(int64_t m, int64_t n, int64_t k) {
+  return (size_t)std::max<int64_t>(mhs_gemm_workspace_bytes(m, n, k), 0);
+}
+
+size_t block_fwd_ws(const BlockDims& s) {
+  return std::max({mhs_scan_fwd_workspace_bytes(s.B, s.T, s.d, s.N), gemm_ws(s.M, 2 * s.d, s.dm),
+                   gemm_ws(s.M, s.P, s.d), gemm_ws(s.M, s.dm, s.d), (size_t)256});
+}
+
+// The backward's buffers: the gated y's gradient (then the conv output's), y's,
+// xz's, the projections', the norm output's, and a part that every launch
+// sequence uses in turn.
+struct BlockBwdWs {
+  size_t dgate, dy, dxz, dproj, dh, part, part_bytes, total;
+};
+
+BlockBwdWs block_bwd_ws(const BlockDims& s) {
+  BlockBwdWs o;
+  size_t off = 0;
+  auto take = [&](size_t floats) {
+    const size_t at = off;
+    off += round_up(floats * 4, 256);
+    return at;
+  };
+  o.dgate = take((size_t)s.M * s.d);
+  o.dy = take((size_t)s.M * s.d);
+  o.dxz = take((size_t)s.M * 2 * s.d);
+  o.dproj = take((size_t)s.M * s.P);
+  o.dh = take((size_t)s.M * s.dm);
+  o.part = off;
+  o.part_bytes = std::max({mhs_scan_bwd_workspace_bytes(s.B, s.T, s.d, s.N, s.chunk),
+                           mhs_out_gate_bwd_workspace_bytes(s.B, s.T, s.d),
+                           mhs_conv1d_silu_bwd_workspace_bytes(s.B, s.T, s.d, s.taps),
+                           mhs_rmsnorm_bwd_workspace_bytes(s.M, s.dm), gemm_ws(s.M, s.d, s.dm),
+                           gemm_ws(s.dm, s.d, s.M), gemm_ws(s.M, s.d, s.P),
+                           gemm_ws(s.P, s.d, s.M), gemm_ws(s.M, s.dm, 2 * s.d),
+                           gemm_ws(2 * s.d, s.dm, s.M), (size_t)256});
+  o.total = off + o.part_bytes;
+  return o;
+}
+
+int check_block_weights(const mhs_block_weights* w) {
+  if (!w) return fail(MHS_EINVAL, "null pointer argument");
+  const void* ps[] = {w->norm_weight, w->in_proj, w->conv_weight, w->conv_bias, w->dt_proj,
+                      w->dt_bias,     w->A,       w->B_proj,      w->C_proj,    w->D_skip,
+                      w->out_proj};
+  for (const void* q : ps) {
+    if (!q) return fail(MHS_EINVAL, "null weight pointer");
+    if (!aligned16(q)) return fail(MHS_EINVAL, "device pointers must be 16-byte aligned");
+  }
+  return MHS_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t mhs_block_saved_bytes(int64_t batch, int64_t seqlen, int64_t d_model, int64_t d_inner,
+                             int64_t d_state, int64_t conv_taps, int64_t chunk, int with_ckpt) {
+  BlockDims s;
+  if (block_dims(batch, seqlen, d_model, d_inner, d_state, conv_taps, chunk, s)) return 0;
+  return block_saved(s, with_ckpt != 0).total;
+}
+
+size_t mhs_block_fwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t d_model,
+                                     int64_t d_inner, int64_t d_state, int64_t conv_taps) {
+  BlockDims s;
+  if (block_dims(batch, seqlen, d_model, d_inner, d_state, conv_taps, 1, s)) return 0;
+  return block_fwd_ws(s);
+}
+
+size_t mhs_block_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t d_model,
+                                     int64_t d_inner, int64_t d_state, int64_t conv_taps,
+                                     int64_t chunk) {
+  BlockDims s;
+  if (block_dims(batch, seqlen, d_model, d_inner, d_state, conv_taps, chunk, s)) return 0;
+  return block_bwd_ws(s).total;
+}
+
+int mhs_block_fwd_f32(const mhs_block_weights* w, const float* x, const float* delta, float* x_out,
+                      float* out, float* xz, void* saved, float* h_last, int64_t batch,
+                      int64_t seqlen, int64_t d_model, int64_t d_inner, int64_t d_state,
+                      int64_t conv_taps, int64_t chunk, int with_ckpt, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+  g_err[0] = '\0';
+  BlockDims s;
+  int rc = block_dims(batch, seqlen, d_model, d_inner, d_state, conv_taps, chunk, s);
+  if (rc) return rc;
+  if ((rc = check_block_weights(w)) != 0) return rc;
+  if (!x || !out || !xz || !saved || !workspace || (delta && !x_out))
+    return fail(MHS_EINVAL, "null pointer argument");
+  if (workspace_bytes < block_fwd_ws(s))
+    return fail(MHS_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes,
+                block_fwd_ws(s));
+  if ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(saved)) & 255u)
+    return fail(MHS_EINVAL, "workspace and saved must be 256-byte aligned");
+  if (!aligned16(xz) || !aligned16(out)) return fail(MHS_EINVAL, "device pointers must be 16-byte aligned");
+  const BlockSaved o = block_saved(s, with_ckpt != 0);
+  auto at = [&](size_t off) { return reinterpret_cast<float*>(static_cast<char*>(saved) + off); };
+  float *h = at(o.h), *xc = at(o.xc), *proj = at(o.proj), *y = at(o.y), *gate = at(o.gate),
+        *wp = at(o.wproj);
+  rc = delta ? mhs_add_rmsnorm_fwd_f32(x, delta, w->norm_weight, x_out, h, at(o.rstd), s.M, s.dm,
+                                       w->eps, stream)
+             : mhs_rmsnorm_fwd_f32(x, w->norm_weight, h, at(o.rstd), s.M, s.dm, w->eps, stream);
+  if (rc) return rc;
+  rc = mhs_gemm_f32(MHS_GEMM_NT, h, s.dm, w->in_proj, s.dm, xz, 2 * s.d, s.M, 2 * s.d, s.dm, 0,
+                    workspace, workspace_bytes, stream);
+  if (rc) return rc;
+  rc = mhs_conv1d_silu_fwd_f32(xz, 2 * s.d, w->conv_weight, w->conv_bias, xc, s.B, s.T, s.d, s.taps,
+                               stream);
+  if (rc) return rc;
+  const long long nd = s.d * s.d / 4, nn = s.N * s.d / 4;
+  hipLaunchKernelGGL(mhs::concat3_kernel<>, dim3((unsigned)((nd + 2 * nn + 255) / 256)), dim3(256),
+                     0, static_cast<hipStream_t>(stream),
+                     reinterpret_cast<const float4*>(w->dt_proj),
+                     reinterpret_cast<const float4*>(w->B_proj),
+                     reinterpret_cast<const float4*>(w->C_proj), reinterpret_cast<float4*>(wp), nd,
+                     nn, nn);
+  if ((rc = check_launch("weight concatenation kernel")) != 0) return rc;
+  rc = mhs_gemm_f32(MHS_GEMM_NT, xc, s.d, wp, s.d, proj, s.P, s.M, s.P, s.d, 0, workspace,
+                    workspace_bytes, stream);
+  if (rc) return rc;
+  rc = mhs_scan_gated_fwd_f32(xc, proj, w->A, proj + s.d, proj + s.d + s.N, w->dt_min, w->dt_max,
+                              w->dt_bias, y, with_ckpt ? at(o.ckpt) : nullptr, h_last, workspace,
+                              workspace_bytes, s.B, s.T, s.d, s.N, s.chunk, s.P, s.P, stream);
+  if (rc) return rc;
+  rc = mhs_out_gate_fwd_f32(y, w->D_skip, xz + s.d, 2 * s.d, gate, s.B, s.T, s.d, stream);
+  if (rc) return rc;
+  return mhs_gemm_f32(MHS_GEMM_NT, gate, s.d, w->out_proj, s.d, out, s.dm, s.M, s.dm, s.d, 0,
+                      workspace, workspace_bytes, stream);
+}
+
+int mhs_block_bwd_f32(const mhs_block_weights* w, const float* x, const float* xz,
+                      const void* saved, const float* dout, const float* dres,
+                      const mhs_block_grads* g, int64_t batch, int64_t seqlen, int64_t d_model,
+                      int64_t d_inner, int64_t d_state, int64_t conv_taps, int64_t chunk,
+                      void* workspace, size_t workspace_bytes, void* stream) {
+  g_err[0] = '\0';
+  BlockDims s;
+  int rc = block_dims(batch, seqlen, d_model, d_inner, d_state, conv_taps, chunk, s);
+  if (rc) return rc;
+  if ((rc = check_block_weights(w)) != 0) return rc;
+  if (!x || !xz || !saved || !dout || !g || !workspace)
+    return fail(MHS_EINVAL, "null pointer argument");
+  for (const void* q : {(const void*)g->x, (const void*)g->norm_weight, (const void*)g->conv_weight,
+                        (const void*)g->conv_bias, (const void*)g->proj, (const void*)g->dt_bias,
+                        (const void*)g->A, (const void*)g->D_skip}) {
+    if (!q) return fail(MHS_EINVAL, "null gradient pointer");
+    if (!aligned16(q)) return fail(MHS_EINVAL, "device pointers must be 16-byte aligned");
+  }
+  const BlockBwdWs b = block_bwd_ws(s);
+  if (workspace_bytes < b.total)
+    return fail(MHS_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, b.total);
+  if ((reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(saved)) & 255u)
+    return fail(MHS_EINVAL, "workspace and saved must be 256-byte aligned");
+  const BlockSaved o = block_saved(s, true);
+  auto at = [&](size_t off) {
+    return reinterpret_cast<const float*>(static_cast<const char*>(saved) + off);
+  };
+  auto ws = [&](size_t off) {
+    return reinterpret_cast<float*>(static_cast<char*>(workspace) + off);
+  };
+  const float *xc = at(o.xc), *proj = at(o.proj);
+  float *dgate = ws(b.dgate), *dy = ws(b.dy), *dxz = ws(b.dxz), *dproj = ws(b.dproj),
+        *dh = ws(b.dh);
+  float* const dxc = dgate;   // the gated y's gradient is spent by then
+  void* const part = ws(b.part);
+  auto gemm = [&](int form, const float* a, int64_t lda, const float* bb, int64_t ldb, float* c,
+                  int64_t m, int64_t n, int64_t k, int acc) {
+    return mhs_gemm_f32(form, a, lda, bb, ldb, c, n, m, n, k, acc, part, b.part_bytes, stream);
+  };
+  if ((rc = gemm(MHS_GEMM_NN, dout, s.dm, w->out_proj, s.d, dgate, s.M, s.d, s.dm, 0)) != 0) return rc;
+  if (g->out_proj &&
+      (rc = gemm(MHS_GEMM_TN, dout, s.dm, at(o.gate), s.d, g->out_proj, s.dm, s.d, s.M, 0)) != 0)
+    return rc;
+  rc = mhs_out_gate_bwd_f32(at(o.y), w->D_skip, xz + s.d, 2 * s.d, dgate, dy, dxz + s.d, 2 * s.d,
+                            g->D_skip, part, b.part_bytes, s.B, s.T, s.d, stream);
+  if (rc) return rc;
+  rc = mhs_scan_gated_bwd_f32(xc, proj, w->A, proj + s.d, proj + s.d + s.N, w->dt_min, w->dt_max,
+                              w->dt_bias, dy, nullptr, at(o.ckpt), dxc, dproj, g->A, dproj + s.d,
+                              dproj + s.d + s.N, g->dt_bias, part, b.part_bytes, s.B, s.T, s.d,
+                              s.N, s.chunk, s.P, s.P, s.P, s.P, stream);
+  if (rc) return rc;
+  if ((rc = gemm(MHS_GEMM_NN, dproj, s.P, at(o.wproj), s.d, dxc, s.M, s.d, s.P, 1)) != 0) return rc;
+  if ((rc = gemm(MHS_GEMM_TN, dproj, s.P, xc, s.d, g->proj, s.P, s.d, s.M, 0)) != 0) return rc;
+  rc = mhs_conv1d_silu_bwd_f32(xz, 2 * s.d, w->conv_weight, w->conv_bias, dxc, dxz, 2 * s.d,
+                               g->conv_weight, g->conv_bias, part, b.part_bytes, s.B, s.T, s.d,
+                               s.taps, stream);
+  if (rc) return rc;
+  if ((rc = gemm(MHS_GEMM_NN, dxz, 2 * s.d, w->in_proj, s.dm, dh, s.M, s.dm, 2 * s.d, 0)) != 0) return rc;
+  if (g->in_proj &&
+      (rc = gemm(MHS_GEMM_TN, dxz, 2 * s.d, at(o.h), s.dm, g->in_proj, 2 * s.d, s.dm, s.M, 0)) != 0)
+    return rc;
+  return mhs_rmsnorm_bwd_f32(dh, x, w->norm_weight, at(o.rstd), dres, g->x, g->norm_weight, part,
+                             b.part_bytes, s.M, s.dm, stream);
 }
 
 }  // extern "C"

@@ -47,7 +47,7 @@ struct GemmArgs {
 
 constexpr int kGemmBK = 16;       // k depth of a tile: one 32x32x16 MFMA
 constexpr int kGemmThreads = 256; // 4 waves
-constexpr int kGemmBM = 128, kGemmBN = 128;
+constexpr int kGemmTile = 128, kGemmSmallTile = 64;
 constexpr int kGemmFlip = 4;      // k tiles between changes of sign (see below)
 constexpr int kGemmPad = 64;      // bytes between the halves of an LDS plane
 
@@ -81,13 +81,20 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8 (&p)[3]) {
   }
 }
 
-// The staging of one operand's R x 16 tile: T tasks per thread, a task being
+// The staging of one operand's R x 16 tile: one task per thread, a task being
 // 8 consecutive k of one row. K-major memory: two 16-byte loads; otherwise
-// eight 4-byte loads, consecutive lanes on consecutive rows.
-template <int R, bool KMAJOR>
+// eight 4-byte loads, consecutive lanes on consecutive rows. R = 128: every
+// thread has a task of each operand; R = 64: the first half of the threads
+// stage A, the second half B (LATE), whole waves.
+template <int R, bool KMAJOR, bool LATE>
 struct GemmLoader {
-  static constexpr int T = R * 2 / kGemmThreads;
-  static_assert(R * 2 % kGemmThreads == 0, "whole tasks");
+  static constexpr int T = 1;
+  static constexpr bool kAll = R * 2 == kGemmThreads;
+  static_assert(kAll || R * 4 == kGemmThreads, "one task of one or of each operand");
+  __device__ __forceinline__ static bool mine() {
+    const int w0 = __builtin_amdgcn_readfirstlane(threadIdx.x);
+    return kAll || (LATE ? w0 >= R * 2 : w0 < R * 2);
+  }
   const float* base;   // of the block's rows, at its first k
   long long ld;
   int width;           // rows from the block's first to the operand's last
@@ -100,12 +107,12 @@ struct GemmLoader {
     base = KMAJOR ? p + (long long)r0 * ld_ + k_first : p + k_first * ld_ + r0;
 #pragma unroll
     for (int i = 0; i < T; ++i) {
-      const int t = threadIdx.x + i * kGemmThreads;
+      const int t = threadIdx.x - (!kAll && LATE ? R * 2 : 0);
       const int row = KMAJOR ? t >> 1 : t % R;
       const int half = KMAJOR ? t & 1 : t / R;
       kpos[i] = 8 * half;
       lds[i] = half * gemm_half_bytes(R) + row * 16;
-      off[i] = r0 + row < rows
+      off[i] = mine() && r0 + row < rows
                    ? (KMAJOR ? 4u * ((unsigned)row * (unsigned)ld_ + 8u * half)
                              : 4u * ((unsigned)(8 * half) * (unsigned)ld_ + (unsigned)row))
                    : kOOB;
@@ -116,6 +123,7 @@ struct GemmLoader {
   // offset; otherwise the resource ends with the last k's row, and ld >=
   // rows puts every later k past its end).
   __device__ __forceinline__ void load(float (&v)[T][8], int kt, int left) const {
+    if (!mine()) return;
     if constexpr (KMAJOR) {
       const GBuf g(base + (long long)kt * kGemmBK, left > 0 ? kOOB - 1u : 0u);
 #pragma unroll
@@ -143,6 +151,7 @@ struct GemmLoader {
     }
   }
   __device__ __forceinline__ void store(char* tile, const float (&w)[T][8], unsigned sign) const {
+    if (!mine()) return;
 #pragma unroll
     for (int i = 0; i < T; ++i) {
       float v[8];
@@ -157,7 +166,8 @@ struct GemmLoader {
   }
 };
 
-// One 128 x 128 tile per block, 2 x 2 waves of 64 x 64, k 16 deep and double
+// One 128 x 128 tile per block, 2 x 2 waves of 64 x 64 (or 64 x 64 of 32 x 32,
+// for products of few tiles), k 16 deep and double
 // buffered: while a wave multiplies a tile it splits the next one into the
 // other buffer and loads the one after it into registers.
 // Bound by the matrix cores at the power limit: per k tile a wave issues 24
@@ -172,9 +182,10 @@ struct GemmLoader {
 // here (1.25). 256 x 128 tiles (two blocks per CU, a quarter fewer LDS reads)
 // were within 4% either way; each k tile's products summed from zero and then
 // added (a third of the error) took 8% longer.
-template <bool AK, bool BK>
-__global__ void __launch_bounds__(kGemmThreads, 3) gemm3_kernel(GemmArgs g) {
-  constexpr int BM = kGemmBM, BN = kGemmBN;
+template <bool AK, bool BK, int TILE>
+__global__ void __launch_bounds__(kGemmThreads, TILE == kGemmTile ? 3 : 4)
+gemm3_kernel(GemmArgs g) {
+  constexpr int BM = TILE, BN = TILE;
   constexpr int FM = BM / 64, FN = BN / 64;   // 32 x 32 fragments per wave
   extern __shared__ float lds_f[];
   char* const lds = reinterpret_cast<char*>(lds_f);
@@ -192,8 +203,8 @@ __global__ void __launch_bounds__(kGemmThreads, 3) gemm3_kernel(GemmArgs g) {
   const int k_len = min(g.K - k_first, g.kt_per_split * kGemmBK);
   const int nk = (k_len + kGemmBK - 1) / kGemmBK;
 
-  const GemmLoader<BM, AK> la(g.A, g.lda, m0, g.M, k_first);
-  const GemmLoader<BN, BK> lb(g.B, g.ldb, n0, g.N, k_first);
+  const GemmLoader<BM, AK, false> la(g.A, g.lda, m0, g.M, k_first);
+  const GemmLoader<BN, BK, true> lb(g.B, g.ldb, n0, g.N, k_first);
   float va[la.T][8], vb[lb.T][8];
   f32x16 acc[FM][FN];
 #pragma unroll
@@ -305,6 +316,18 @@ __global__ void __launch_bounds__(kGemmThreads, 3) gemm3_kernel(GemmArgs g) {
       }
     }
   }
+}
+
+// out = the rows of a, then b, then c: float4s, na + nb + nc of them.
+template <int UNUSED = 0>
+__global__ void __launch_bounds__(256)
+concat3_kernel(const float4* __restrict__ a, const float4* __restrict__ b,
+               const float4* __restrict__ c, float4* __restrict__ out, long long na, long long nb,
+               long long nc) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i < na) out[i] = a[i];
+  else if (i < na + nb) out[i] = b[i - na];
+  else if (i < na + nb + nc) out[i] = c[i - na - nb];
 }
 
 // out (M, N; rows ldc apart) = the sum of the split-K partials (splits, M,

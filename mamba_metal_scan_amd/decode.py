@@ -15,6 +15,7 @@ import torch
 import torch.nn as nn
 
 from . import _native
+from .block import plain, plain_mods
 from .linear import no_hooks
 
 # mhs_decode_layer: 13 pointers, the conv window's strides, the next window,
@@ -23,12 +24,6 @@ _LAYER = struct.Struct("13Q3qQ4f")
 
 
 _f32 = torch.float32
-
-
-def _plain(t: Optional[torch.Tensor], dev: torch.device, shape: tuple) -> bool:
-    """Whether t is fp32 of that shape, contiguous, on dev."""
-    return (t is not None and t.dtype is _f32 and t.shape == shape and t.device == dev
-            and t.is_contiguous())
 
 
 def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: tuple,
@@ -43,10 +38,8 @@ def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: 
             m["norm"], m["in_proj"], m["conv"], m["dt_proj"], m["B_proj"], m["C_proj"],
             m["out_proj"])
         h, win = bc["h"], bc["conv"]
-        for mod, kind in zip(mods, kinds):
-            if (type(mod) is not kind or mod._forward_hooks or mod._forward_pre_hooks
-                    or mod._backward_hooks or mod._backward_pre_hooks):
-                return None
+        if not plain_mods(mods, kinds):
+            return None
         w_dt, w_conv = dt_proj._parameters, conv._parameters
         weights = (norm._parameters["weight"], in_proj._parameters["weight"], w_conv["weight"],
                    w_conv["bias"], w_dt["weight"], w_dt["bias"], p["A"],
@@ -54,10 +47,10 @@ def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: 
                    out_proj._parameters["weight"], h)
         biases = (in_proj._parameters["bias"], b_proj._parameters["bias"],
                   c_proj._parameters["bias"], out_proj._parameters["bias"])
-    except KeyError:
+    except (KeyError, AttributeError):
         return None
     for t, shape in zip(weights, shapes):
-        if not _plain(t, dev, shape):
+        if not plain(t, dev, shape):
             return None
     if (any(v is not None for v in biases) or win is None or win.dtype is not _f32
             or win.shape != shapes[12] or win.device != dev or not norm.hip
@@ -96,7 +89,7 @@ def decode_step(model: nn.Module, x: torch.Tensor, cache: dict) -> Optional[torc
             or d_model % 4 or d % 4 or not 2 <= taps <= 8 or not 1 <= n <= 64 or batch > 65535):
         return None
     head_w, norm_w = head._parameters.get("weight"), ln_f._parameters.get("weight")
-    if (not _plain(norm_w, dev, (d_model,)) or not _plain(head_w, dev, (head.out_features, d_model))
+    if (not plain(norm_w, dev, (d_model,)) or not plain(head_w, dev, (head.out_features, d_model))
             or (head_w.data_ptr() | norm_w.data_ptr() | x.data_ptr()) & 15):
         return None
     windows = torch.empty((len(blocks), batch, d, taps - 1), dtype=torch.float32,

@@ -38,6 +38,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ._native import rmsnorm_supported
+from .block import BlockHIP, block_forward, block_params
 from .conv import conv1d_silu
 from .decode import decode_step
 from .fused import mamba_inner, out_gate, selective_scan_gated
@@ -176,6 +177,19 @@ def parallel_scan(a: torch.Tensor, b: torch.Tensor, chunk: int = 0) -> torch.Ten
 
 # ------------------------------------------------------------------ the block
 
+def _conv_tail(xt: torch.Tensor, k: int) -> torch.Tensor:
+    """The last k - 1 inputs (zeros before the first) of a conv of k taps over
+    xt (B, d_inner, T): the window a recurrent cache keeps."""
+    tail = xt[:, :, -(k - 1):]
+    return F.pad(tail, (k - 1 - tail.shape[2], 0)) if tail.shape[2] < k - 1 else tail
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """t, contiguous and 16-byte aligned."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() & 15 else t
+
+
 class MambaBlock(nn.Module):
     """Gated causal depthwise conv + diagonal selective SSM, with a residual."""
 
@@ -283,7 +297,43 @@ class MambaBlock(nn.Module):
         return (self._fused(xz) and self.d_inner % 4 == 0 and self.A.shape[1] % 4 == 0
                 and self.conv.kernel_size[0] <= 8)
 
+    def _native(self, x, delta=None, cache=None):
+        """(x + delta (or x), the block's output without its residual add) as
+        one native call per direction, or None where that does not apply:
+        fp32 ROCm tensors outside autocast and tracing, with a norm, in_proj
+        and out_proj that are plain modules (the other modules' weights are
+        read directly, as in the fused path). With a cache (a prefill, without
+        autograd) it is filled."""
+        norm = self._modules["norm"]
+        if (type(self) is not MambaBlock or self.scan_impl == "torch" or type(norm) is not RMSNorm
+                or not norm.uses_hip(x) or x.dim() != 3 or not no_hooks(norm)
+                or torch.is_autocast_enabled() or torch.compiler.is_compiling()):
+            return None
+        grad = torch.is_grad_enabled()
+        if cache is not None and (grad or (cache.get("h") is not None and x.shape[1] == 1)):
+            return None
+        params = block_params(self, x, strict=cache is not None)
+        if params is None:
+            return None
+        x = _aligned(x)
+        if delta is not None:
+            if delta.shape != x.shape or delta.dtype != x.dtype or delta.device != x.device:
+                return None
+            delta = _aligned(delta)
+        consts = (norm.eps, self.dt_min, self.dt_max, self.ckpt_chunk)
+        if grad:
+            return BlockHIP.apply(x, delta, consts, *params)
+        x_out, out, xz, _, h = block_forward(x, delta, params, consts, False, cache is not None)
+        if cache is not None:
+            k = self.conv.kernel_size[0]
+            cache["conv"] = _conv_tail(xz[..., :self.d_inner].transpose(1, 2), k)
+            cache["h"] = h
+        return x_out, out
+
     def forward(self, x, cache=None):
+        r = self._native(x, None, cache)
+        if r is not None:
+            return r[0] + r[1]
         if self.norm.uses_hip(x):
             # x itself, and its norm; the backward adds x's two gradients in
             # the norm's kernel.
@@ -309,10 +359,7 @@ class MambaBlock(nn.Module):
             xt = x.transpose(1, 2)                                       # (B, d_inner, T)
             x = self._conv_silu(x)
             if cache is not None:
-                tail = xt[:, :, -(k - 1):]
-                if tail.shape[2] < k - 1:
-                    tail = F.pad(tail, (k - 1 - tail.shape[2], 0))
-                cache["conv"] = tail
+                cache["conv"] = _conv_tail(xt, k)
             y, h_last = self._scan(x, return_state=True)
             if cache is not None:
                 cache["h"] = h_last
@@ -368,6 +415,10 @@ class TinyMamba(nn.Module):
             # called as block(x, cache) in the loop below).
             delta = None
             for block, bc in zip(self.blocks, caches):
+                r = block._native(x, delta, bc)
+                if r is not None:
+                    x, delta = r
+                    continue
                 if delta is None:
                     x, h = rms_norm_residual(x, block.norm.weight, block.norm.eps)
                 else:

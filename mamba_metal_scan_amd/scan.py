@@ -82,9 +82,27 @@ def _hip_device(t: torch.Tensor) -> bool:
     return t.is_cuda and torch.version.hip is not None
 
 
+def _takes(x, dt, aneg, b_in, c_in, chunk) -> bool:
+    """Whether _validate accepts the arguments, by direct comparisons (an eager
+    call's host time counts where the kernels take a few microseconds)."""
+    if not (x.is_cuda and torch.version.hip is not None and x.dim() == 3 and aneg.dim() == 2
+            and type(chunk) is int and chunk >= 1):
+        return False
+    dtype, dev, shape = x.dtype, x.device, x.shape
+    d, n = aneg.shape
+    bc = (shape[0], shape[1], n)
+    return ((dtype is torch.float32 or dtype is torch.bfloat16) and dt.dtype is dtype
+            and b_in.dtype is dtype and c_in.dtype is dtype and aneg.dtype is torch.float32
+            and dt.shape == shape and shape[2] == d and b_in.shape == bc and c_in.shape == bc
+            and dt.device == dev and aneg.device == dev and b_in.device == dev
+            and c_in.device == dev and (n == 0 or _native.preferred_chunk(n) != 0))
+
+
 def _validate(x, dt, aneg, b_in, c_in, chunk) -> None:
     """Argument checks in the reference's order and exception types
     (mamba_metal/scan.py:344-365, :274-276)."""
+    if not torch.compiler.is_compiling() and _takes(x, dt, aneg, b_in, c_in, chunk):
+        return
     tensors = (x, dt, aneg, b_in, c_in)
     if not all(_hip_device(t) for t in tensors):
         raise RuntimeError("scan_impl='hip' needs every input on the ROCm device; saw devices "
@@ -133,8 +151,12 @@ class SelectiveScanHIP(torch.autograd.Function):
             ctx.save_for_backward(x, dt, aneg, b_in, c_in)
         else:
             need_grad = any(ctx.needs_input_grad[:5])
-            y, ckpt, h_last = _native.dispatch("scan_fwd")(x, dt, aneg, b_in, c_in, chunk,
-                                                           need_grad)
+            if torch.compiler.is_compiling():
+                y, ckpt, h_last = _native.dispatch("scan_fwd")(x, dt, aneg, b_in, c_in, chunk,
+                                                               need_grad)
+            else:   # no final state that nobody asked for
+                y, ckpt, h_last = _native.scan_fwd_into(x, dt, aneg, b_in, c_in, chunk,
+                                                        need_grad, return_state)
             ctx.save_for_backward(x, dt, aneg, b_in, c_in, ckpt)
         if return_state:
             return y, h_last
@@ -216,10 +238,12 @@ def selective_state_step(h: torch.Tensor, x: torch.Tensor, dt: torch.Tensor,
     The same update as the reference's recurrent step (mamba_metal/model.py:234-241)
     in one kernel. Not differentiable (it mutates h); for inference.
     """
-    tensors = (h, x, dt, aneg, b_in, c_in)
-    if not all(_hip_device(t) for t in tensors):
+    if not (h.is_cuda and x.is_cuda and dt.is_cuda and aneg.is_cuda and b_in.is_cuda
+            and c_in.is_cuda and torch.version.hip is not None):
         raise RuntimeError("selective_state_step needs every input on the ROCm device")
-    if not all(t.dtype == torch.float32 for t in tensors):
+    f32 = torch.float32
+    if not (h.dtype is f32 and x.dtype is f32 and dt.dtype is f32 and aneg.dtype is f32
+            and b_in.dtype is f32 and c_in.dtype is f32):
         raise RuntimeError("selective_state_step is fp32-only")
     bt, d, n = h.shape
     if (x.shape != (bt, d) or dt.shape != (bt, d) or aneg.shape != (d, n)

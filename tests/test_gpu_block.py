@@ -1,0 +1,158 @@
+"""GPU parity of the native block (mhs_block_fwd_f32 / _bwd_f32): a MambaBlock's
+output, input gradient and every parameter gradient, and a prefill's cache,
+against the float64 torch block (scan_impl 'torch', the reference's own
+forward, mamba_metal/model.py:225-256).
+
+Bar: 1e-4 max relative per tensor, the build's parity bar.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import assert_close
+from mamba_metal_scan_amd import block as block_mod
+from mamba_metal_scan_amd.model import MambaBlock, MambaConfig, TinyMamba
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _blocks(d_model, d_inner, n=16, k=4, chunk=16):
+    kw = dict(vocab_size=8, d_model=d_model, d_state=n, d_conv=k, ckpt_chunk=chunk)
+    torch.manual_seed(d_model + d_inner + n)
+    hip = MambaBlock(MambaConfig(scan_impl="hip", **kw), d_inner)
+    with torch.no_grad():
+        hip.dt_proj.bias.normal_()
+        hip.D_skip.normal_()
+        hip.A.normal_(0.0, 3.0)
+        hip.norm.weight.normal_(1.0, 0.1)
+    ref = MambaBlock(MambaConfig(scan_impl="torch", **kw), d_inner).double()
+    ref.load_state_dict({k2: v.double() for k2, v in hip.state_dict().items()})
+    return hip.to(DEV), ref
+
+
+def _calls(monkeypatch):
+    """The native forwards, by whether they kept checkpoints."""
+    seen = []
+    real = block_mod.block_forward
+
+    def spy(*args):
+        seen.append(args[4])
+        return real(*args)
+    monkeypatch.setattr(block_mod, "block_forward", spy)
+    monkeypatch.setattr("mamba_metal_scan_amd.model.block_forward", spy)
+    return seen
+
+
+# Rows and widths below, at and above the products' tiles (64, 128), sequences
+# of one step, of a chunk's remainder and in time segments, every conv length's
+# ends, strides that recompute checkpoints.
+@pytest.mark.parametrize("bt,t,d_model,d_inner,n,k,chunk", [
+    (1, 1, 4, 4, 4, 4, 16), (2, 5, 64, 68, 16, 1, 16), (3, 65, 128, 132, 8, 8, 64),
+    (2, 300, 132, 64, 64, 4, 32), (4, 129, 68, 256, 16, 2, 100)])
+def test_forward_and_gradients(monkeypatch, bt, t, d_model, d_inner, n, k, chunk):
+    print(f"[case] block {bt}x{t} {d_model} {d_inner} {n} {k} {chunk}", flush=True)
+    hip, ref = _blocks(d_model, d_inner, n, k, chunk)
+    seen = _calls(monkeypatch)
+    g = torch.Generator().manual_seed(t)
+    x, dy = (torch.randn(bt, t, d_model, generator=g) for _ in range(2))
+    xr, xh = x.double().requires_grad_(), x.to(DEV).requires_grad_()
+    yr, yh = ref(xr), hip(xh)
+    yr.backward(dy.double())
+    yh.backward(dy.to(DEV))
+    torch.cuda.synchronize()
+    assert seen == [True]
+    assert_close("out", yh, yr)
+    assert_close("dx", xh.grad, xr.grad)
+    for (name, p), q in zip(hip.named_parameters(), ref.parameters()):
+        assert_close(name, p.grad, q.grad)
+
+
+@pytest.mark.parametrize("t", [1, 2, 3, 40])
+def test_prefill_fills_the_cache(monkeypatch, t):
+    """Prompts shorter and longer than the conv window."""
+    hip, ref = _blocks(64, 96)
+    seen = _calls(monkeypatch)
+    x = torch.randn(3, t, 64, generator=torch.Generator().manual_seed(t))
+    ch, cr = {}, {}
+    with torch.no_grad():
+        yh, yr = hip(x.to(DEV), ch), ref(x.double(), cr)
+    torch.cuda.synchronize()
+    assert seen == [False]
+    assert_close("out", yh, yr)
+    assert_close("h", ch["h"], cr["h"])
+    assert_close("conv", ch["conv"], cr["conv"])
+
+
+def test_frozen_weights_and_unused_outputs():
+    """Products whose gradient nobody asks for are left out; the gradient of x
+    + delta alone (the block's output unused) passes through."""
+    hip, _ = _blocks(64, 96)
+    x = torch.randn(2, 33, 64, generator=torch.Generator().manual_seed(0)).to(DEV)
+
+    def run(frozen):
+        for name, p in hip.named_parameters():
+            p.requires_grad_(name not in frozen)
+            p.grad = None
+        xi = x.clone().requires_grad_()
+        hip(xi).square().sum().backward()
+        return xi.grad, {k: p.grad for k, p in hip.named_parameters()}
+    dx, full = run(())
+    for frozen in (("in_proj.weight", "out_proj.weight"), ("A", "dt_proj.weight")):
+        dx2, part = run(frozen)
+        assert torch.equal(dx, dx2)
+        for k, v in part.items():
+            assert (v is None) if k in frozen else torch.equal(v, full[k]), k
+    xi = x.clone().requires_grad_()
+    delta = torch.ones_like(x).requires_grad_()
+    x_out, _ = hip._native(xi, delta)
+    x_out.sum().backward()
+    assert torch.equal(xi.grad, torch.ones_like(x)) and torch.equal(delta.grad, xi.grad)
+
+
+def test_hooks_subclasses_and_offset_views_take_the_module_path(monkeypatch):
+    hip, ref = _blocks(64, 96)
+    seen = _calls(monkeypatch)
+    x = torch.randn(2, 20, 64, generator=torch.Generator().manual_seed(5))
+    want = ref(x.double())
+    ran = []
+    h = hip.out_proj.register_forward_hook(lambda m, i, o: ran.append(1))
+    assert_close("hook", hip(x.to(DEV)), want)
+    h.remove()
+    assert ran == [1] and seen == []
+
+    class Doubled(MambaBlock):
+        def mix(self, h, cache=None):
+            return 2 * super().mix(h, cache)
+    hip.__class__ = Doubled
+    assert_close("subclass", hip(x.to(DEV)) - x.to(DEV), 2 * (want - x.double()))
+    hip.__class__ = MambaBlock
+    assert seen == []
+    buf = torch.empty(x.numel() + 1, device=DEV)   # x 4 bytes into its storage: copied
+    view = buf[1:].view(x.shape).copy_(x.to(DEV))
+    assert_close("offset view", hip(view), want)
+    assert seen == [True]
+
+
+def test_model_gradients_equal_the_module_path():
+    """A TinyMamba's loss and gradients through the native blocks against the
+    same model with a hook on every in_proj (the module path)."""
+    torch.manual_seed(0)
+    m = TinyMamba(MambaConfig(vocab_size=203, d_model=64, n_layers=3, d_ff=128,
+                              scan_impl="hip")).to(DEV)
+    idx = torch.randint(0, 203, (3, 50), generator=torch.Generator().manual_seed(2)).to(DEV)
+
+    def grads():
+        m.zero_grad(set_to_none=True)
+        _, loss = m(idx[:, :-1], idx[:, 1:])
+        loss.backward()
+        return loss.detach(), {k: p.grad.clone() for k, p in m.named_parameters()}
+    loss, native = grads()
+    handles = [b.in_proj.register_forward_hook(lambda mod, i, o: None) for b in m.blocks]
+    loss2, module = grads()
+    for h in handles:
+        h.remove()
+    assert_close("loss", loss, loss2, tol=1e-6)
+    for k in native:
+        assert_close(k, native[k], module[k], tol=2e-5)
