@@ -303,14 +303,9 @@ bwd_kernel(BwdArgs a) {
     const float* dhl = a.dh_last != nullptr ? a.dh_last + (size_t)b * slice : a.aneg;
     load_states<NPL>(u, GBuf(dhl, a.dh_last != nullptr ? slice_bytes : 0u), st_lane, nvalid,
                      sw);
-    for (int s2 = a.nunits - 1; s2 >= (seg + 1) * a.cunits; --s2) {
-      float lv[NPL];
-      const size_t slot = (size_t)s2 * a.batch + b;
-      load_states<NPL>(lv, GBuf(a.carryL + slot * slice, slice_bytes), st_lane, nvalid, sw);
-      const float sdt = act ? a.carrySdt[slot * D + d] : 0.f;
-#pragma unroll
-      for (int j = 0; j < NPL; ++j) u[j] = __builtin_fmaf(exp2_hw(sdt * a2[j]), u[j], lv[j]);
-    }
+    fold_carries<NPL>(u, a2, a.carryL, a.carrySdt, a.nunits - 1, -1,
+                      a.nunits - (seg + 1) * a.cunits, a.batch, b, slice, st_lane, nvalid, sw, D,
+                      d);
   }
   // u (dh_last) and Aneg come from loads before the walk.
 #pragma unroll

@@ -85,6 +85,7 @@ bool atomic_reduction(bool segmented) {
 constexpr int kDefaultCUs = 256; // MI355X compute units (used when no device can be queried)
 constexpr int kMaxDevices = 64;
 constexpr int kMaxSegments = 8;
+constexpr int kMaxG = 8;          // waves per block
 constexpr int kMinSegChunks = 8; // automatic split: at least 8 chunks per segment
 
 // Forced compute-unit count (0 = query the device); see mhs_set_cu_count.
@@ -118,7 +119,8 @@ int device_cus() {
 
 // Time segments for this shape (see FwdArgs in mhs_fwd.hpp and BwdArgs in
 // mhs_bwd.hpp), in units of nch chunks (16-step sub-chunks in the forward,
-// the backward's chunks in the backward). Automatic: one segment while the
+// the backward's chunks in the backward). Forced, or automatic for grids of
+// about a block per CU (sparser ones: least_segments): one segment while the
 // grid has at least two blocks per CU; below that, enough segments for about
 // per_cu blocks per CU, each at least kMinSegChunks chunks long: the
 // forward's carry pass costs more of its main pass than the backward's does,
@@ -176,12 +178,124 @@ Segments segments_for(int64_t batch, int64_t D, int nch, int per_cu, bool carrie
   return r;
 }
 
+// Plan shape of d_state N: states per lane and waves per block (false: none).
+bool plan_shape(int N, int& npl, int& G) {
+  if (N < 1 || N > MHS_MAX_DSTATE) return false;
+  const int forced = g_npl_override.load(std::memory_order_relaxed);
+  // Automatic: two states per lane up to d_state 32 (more, thinner blocks),
+  // four beyond. One state per lane: the instantiated plans pad d_state to 8
+  // or 16.
+  npl = forced != 0 ? forced : N <= 32 ? 2 : 4;
+  G = npl == 1 ? (N <= 8 ? 4 : N <= 16 ? 8 : 0) : (N + 2 * npl - 1) / (2 * npl);
+  return G >= 1 && G <= kMaxG;
+}
+
+// Time of a pass's grid in us: nb blocks of `chunks` chunks each, resident at
+// most `res` per CU; a chunk takes `alone` us on a CU of one block and
+// `each` us per block on a full one, a round of blocks `base` us more.
+struct PassRate {
+  int res;
+  double alone, each, base;
+  double us(double nb, double chunks, int cus) const {
+    const double full = std::floor(nb / ((double)cus * res)), rem = nb - full * cus * res;
+    double t = full * (chunks * std::max(alone, each * res) + base);
+    if (rem > 0) t += chunks * std::max(alone, each * std::ceil(rem / cus)) + base;
+    return t;
+  }
+};
+
+// The split of a grid that leaves CUs without a block: segments and carry
+// units whose estimated time is the least (their walks, the carry pass, and
+// the fold of the units' carries at each segment's start, 0.2 us a unit,
+// more with several blocks per CU). The rates are those of MI355X at d_state
+// 16 and 64; the estimate was within 10% of the time of 200 measured splits
+// (2 to 210 blocks of 8 to 472 chunks) and its least within 2% of the
+// fastest on average (10% at worst). Against a limit of 8 segments of at
+// least 8 chunks, forward / backward us (GPU time):
+//   1x6664x64x16     109 -> 34 / 199 -> 44     1x1365x64x16  30 -> 20 / 48 -> 24
+//   2x7550x168x16     92 -> 47 / 162 -> 73     1x509x856x16  21 -> 18 / 32 -> 27
+//   4x1024x1024x64   136 -> 109 / 281 -> 216   3x1299x1924x64 266 -> 182 / 483 -> 445
+//   10x5749x666x16  (291) / 610 -> 505         3x1001x1432x16 bf16 (47) / 95 -> 76
+constexpr int kMaxAutoSegments = 64, kMaxAutoUnits = 128;
+
+Segments least_segments(int64_t blocks, int nch, int cus, int npl, int G, bool fwd,
+                        double unit_bytes) {
+  const double w = G * npl / 8.0;   // a block's VALU work against d_state 16's
+  const bool two = npl <= 2;
+  PassRate main, carry;
+  if (fwd) {
+    main = {two ? std::max(1, 16 / G) : 1, two ? 0.97 : 2.2, 0.5 * w, 3.5};
+    carry = {two ? std::max(1, 20 / G) : 1, two ? 0.62 : 1.4, 0.3 * w, 3.5};
+  } else {
+    main = {two ? std::max(1, 12 / G) : 1, two ? 2.1 : 5.3, 1.08 * w, 4.5};
+    carry = {two ? std::max(1, 16 / G) : 2, two ? 0.75 : 1.6, 0.33 * w, 4.5};
+  }
+  const double launch = fwd ? 3 : 6;   // the carry pass's, and the zero fill's
+  Segments best;
+  double least = 0;
+  for (const int ns : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, kMaxAutoSegments}) {
+    if (ns > 1 && nch / ns < 2) break;
+    for (int cu = 1; cu <= 16 && (cu == 1 || (ns > 1 && nch / ns / cu >= 2)); cu *= 2) {
+      Segments r;
+      const int cps = (nch + ns - 1) / ns;
+      r.ups = (cps + cu - 1) / cu;
+      r.cunits = cu;
+      r.cps = r.ups * cu;
+      r.nseg = (nch + r.cps - 1) / r.cps;
+      r.nunits = (nch + r.ups - 1) / r.ups;
+      const double carried = (double)(r.nseg - 1) * cu;
+      if (carried > kMaxAutoUnits || carried * unit_bytes + 512 > MHS_NOALLOC_SCRATCH_BYTES)
+        continue;
+      double us = main.us((double)blocks * r.nseg, r.cps, cus);
+      if (r.nseg > 1)
+        us += carry.us(blocks * carried, r.ups, cus) + launch +
+              0.2 * carried * std::max(1.0, (double)blocks * r.nseg / (2.0 * cus));
+      if (least == 0 || us < least) {
+        least = us;
+        best = r;
+      }
+    }
+  }
+  if (best.nseg == 1) {   // no carries
+    best.cunits = 1;
+    best.ups = best.cps = nch;
+    best.nunits = 1;
+  }
+  return best;
+}
+
+// least_segments for a pass over (batch, D, N), or nothing where the split by
+// blocks per CU (segments_for) stands: forced splits, grids of a block per CU
+// or more, and forwards of up to 32 states from a quarter of that on (there
+// the two were within 4%). The last answers are kept per thread: the search
+// takes about 2 us, and a call asks up to three times.
+bool sparse_segments(int64_t batch, int64_t D, int64_t N, int nch, bool fwd, Segments& out) {
+  if (g_seg_override.load(std::memory_order_relaxed) != 0) return false;
+  const int64_t blocks = batch * ((D + mhs::kCH - 1) / mhs::kCH);
+  const int cus = device_cus();
+  int npl = 0, G = 0;
+  if (blocks >= cus || !plan_shape((int)N, npl, G)) return false;
+  if (fwd && npl <= 2 && 4 * blocks >= cus) return false;
+  struct Entry { int64_t batch, D; int N, nch, cus, npl; bool fwd; Segments s; };
+  thread_local Entry memo[8] = {};
+  thread_local int next = 0;
+  for (const Entry& e : memo)
+    if (e.batch == batch && e.D == D && e.N == N && e.nch == nch && e.cus == cus &&
+        e.npl == npl && e.fwd == fwd) {
+      out = e.s;
+      return true;
+    }
+  out = least_segments(blocks, nch, cus, npl, G, fwd, (double)batch * D * (N + 1) * 4);
+  memo[next] = Entry{batch, D, (int)N, nch, cus, npl, fwd, out};
+  next = (next + 1) % 8;
+  return true;
+}
+
 using FwdFn = void (*)(mhs::FwdArgs);
 using BwdFn = void (*)(mhs::BwdArgs);
 
 constexpr int kKI = mhs::kSteps;           // backward register window (steps)
 constexpr int kMaxLdsBytes = 160 * 1024;   // gfx950 LDS per workgroup
-constexpr int kMaxG = 8;                   // waves per block
 
 // The kernels of one plan for one activation element type.
 struct Kernels {
@@ -290,10 +404,10 @@ bool fill_g1(int G, Plan& p) {
   return true;
 }
 
-bool plan_for(int N, int npl, Plan& p) {
-  // One state per lane: the instantiated plans pad d_state to 8 or 16.
-  const int G = npl == 1 ? (N <= 8 ? 4 : N <= 16 ? 8 : 0) : (N + 2 * npl - 1) / (2 * npl);
-  if (G < 1 || G > kMaxG) return false;
+// Resolve the kernel variant for d_state N. Returns false if unsupported.
+bool make_plan(int N, Plan& p) {
+  int npl = 0, G = 0;
+  if (!plan_shape(N, npl, G)) return false;
   const bool ok = npl == 2 ? fill_g<2>(G, p) : npl == 4 ? fill_g<4>(G, p)
                   : npl == 1 ? fill_g1(G, p) : false;
   if (!ok) return false;
@@ -301,16 +415,6 @@ bool plan_for(int N, int npl, Plan& p) {
   p.G = G;
   p.bwd_ki = kKI;
   return p.fwd_lds <= kMaxLdsBytes && p.bwd_lds <= kMaxLdsBytes && p.bwd_sw_lds <= kMaxLdsBytes;
-}
-
-// Resolve the kernel variant for d_state N. Returns false if unsupported.
-bool make_plan(int N, Plan& p) {
-  if (N < 1 || N > MHS_MAX_DSTATE) return false;
-  const int forced = g_npl_override.load(std::memory_order_relaxed);
-  if (forced != 0) return plan_for(N, forced, p);
-  // Automatic: two states per lane up to d_state 32 (more, thinner blocks),
-  // four beyond.
-  return plan_for(N, N <= 32 ? 2 : 4, p);
 }
 
 // Dynamic-LDS opt-in, once per kernel function.
@@ -439,7 +543,8 @@ WsLayout ws_layout(int64_t batch, int64_t T, int64_t D, int64_t N, int64_t chunk
   const int km = sweep_km(chunk, T, bwd_ki);
   // Segments of the walk's chunks, the same as at stride bwd_ki (a segment
   // of the swept kernel may start inside a caller chunk).
-  w.sg = segments_for(batch, D, (int)((T + kb - 1) / kb), kBwdBlocksPerCU);
+  if (!sparse_segments(batch, D, N, (int)((T + kb - 1) / kb), /*fwd=*/false, w.sg))
+    w.sg = segments_for(batch, D, (int)((T + kb - 1) / kb), kBwdBlocksPerCU);
   w.nseg = w.sg.nseg;
   w.atomic = atomic_reduction(w.nseg > 1);
   size_t off = 0;
@@ -526,7 +631,9 @@ struct FwdWs {
 
 FwdWs fwd_ws_layout(int64_t batch, int64_t T, int64_t D, int64_t N) {
   FwdWs w;
-  w.sg = segments_for(batch, D, (int)((T + mhs::kSteps - 1) / mhs::kSteps), kFwdBlocksPerCU);
+  const int nch = (int)((T + mhs::kSteps - 1) / mhs::kSteps);
+  if (!sparse_segments(batch, D, N, nch, /*fwd=*/true, w.sg))
+    w.sg = segments_for(batch, D, nch, kFwdBlocksPerCU);
   if (w.sg.nseg > 1) {   // carries of the units of segments 0..nseg-2
     const size_t units = (size_t)(w.sg.nseg - 1) * w.sg.cunits;
     w.carryH = 0;

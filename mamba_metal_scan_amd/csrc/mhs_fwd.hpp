@@ -326,14 +326,8 @@ fwd_kernel(FwdArgs a) {
     load_states<NPL>(h, GBuf(a.h_init + ((size_t)b * a.init_nchunk + t_beg / a.init_K - 1) *
                                             ck_stride, slice_bytes), ck_lane, nvalid);
   } else if (!FCARRY && seg > 0 && a.carryH != nullptr) {
-    for (int s2 = 0; s2 < seg * a.cunits; ++s2) {
-      const size_t slot = (size_t)s2 * a.batch + b;
-      float hv[NPL];
-      load_states<NPL>(hv, GBuf(a.carryH + slot * ck_stride, slice_bytes), ck_lane, nvalid);
-      const float sdt = act ? a.carrySdt[slot * D + d] : 0.f;
-#pragma unroll
-      for (int j = 0; j < NPL; ++j) h[j] = __builtin_fmaf(exp2_hw(sdt * a2[j]), h[j], hv[j]);
-    }
+    fold_carries<NPL>(h, a2, a.carryH, a.carrySdt, 0, 1, seg * a.cunits, a.batch, b, ck_stride,
+                      ck_lane, nvalid, 0, D, d);
   }
 #pragma unroll
   for (int j = 0; j < NPL; ++j) h[j] = opaque_copy(h[j]);   // h may come from a load

@@ -1,0 +1,89 @@
+"""The automatic split of sparse grids into many time segments: outputs and
+gradients against the same kernels unsegmented, over the forms the entry
+points take (d_state of each plan, strides that walk, sweep or recompute, bf16,
+the gated scan with strided projections and a bias, a final-state gradient).
+
+Bar: 1e-5 max relative per tensor (fp32 sums in another order; a segment's
+start state is folded from its predecessors' instead of walked), bf16 outputs
+1e-2 (their rounding).
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from helpers import rel_err
+from mamba_metal_scan_amd import _native, selective_scan_gated, selective_scan_hip
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _grads(out, leaves, seed):
+    g = torch.Generator().manual_seed(seed)
+    outs = [o for o in out if o is not None]
+    ups = [torch.randn(o.shape, generator=g).to(DEV, o.dtype) for o in outs]
+    return [o.detach() for o in outs] + list(torch.autograd.grad(outs, leaves, ups))
+
+
+def _both(run):
+    auto = run()
+    _native.set_time_segments(1)
+    try:
+        return auto, run()
+    finally:
+        _native.set_time_segments(0)
+
+
+def _compare(auto, one, bf16):
+    for i, (a, b) in enumerate(zip(auto, one)):
+        tol = 1e-2 if bf16 and a.dtype == torch.bfloat16 else 1e-5
+        assert rel_err(a.float(), b.float()) <= tol, i
+
+
+def _more_workspace(bt, t, d, n):
+    """The split the shape gets is automatic and not the unsegmented one."""
+    need = _native.library().mhs_scan_fwd_workspace_bytes(bt, t, d, n)
+    assert 0 < need <= _native.NOALLOC_SCRATCH_BYTES
+    return need
+
+
+@pytest.mark.parametrize("bt,t,d,n,chunk,bf16", [
+    (1, 577, 64, 16, 16, False), (2, 1000, 40, 5, 32, False), (1, 3001, 33, 64, 100, False),
+    (1, 4099, 70, 16, 64, True), (3, 333, 96, 4, 16, True), (1, 2048, 512, 32, 48, False),
+    (4, 1024, 1024, 64, 16, False)])
+def test_many_segments_equal_one(bt, t, d, n, chunk, bf16):
+    print(f"[case] segments {bt}x{t}x{d}x{n} chunk {chunk} bf16 {bf16}", flush=True)
+    assert _more_workspace(bt, t, d, n) > 0
+    g = torch.Generator().manual_seed(t + d + n)
+    dtype = torch.bfloat16 if bf16 else torch.float32
+
+    def rand(*s):
+        return torch.randn(*s, generator=g)
+    leaves = [rand(bt, t, d).to(DEV, dtype), F.softplus(rand(bt, t, d) - 4).to(DEV, dtype),
+              (0.05 + torch.rand(d, n, generator=g)).to(DEV), rand(bt, t, n).to(DEV, dtype),
+              rand(bt, t, n).to(DEV, dtype)]   # slow decays: carries matter
+    leaves = [v.requires_grad_() for v in leaves]
+
+    def run():
+        return _grads(selective_scan_hip(*leaves, chunk=chunk, return_state=True), leaves, 1)
+    _compare(*_both(run), bf16)
+
+
+def test_gated_scan_in_many_segments():
+    bt, t, d, n = 1, 1500, 68, 16
+    print(f"[case] gated segments {bt}x{t}x{d}x{n}", flush=True)
+    assert _more_workspace(bt, t, d, n) > 0
+    g = torch.Generator().manual_seed(3)
+    proj = torch.randn(bt, t, d + 2 * n, generator=g).to(DEV).requires_grad_()
+    x = torch.randn(bt, t, d, generator=g).to(DEV).requires_grad_()
+    a = torch.randn(d, n, generator=g).to(DEV).requires_grad_()
+    bias = torch.randn(d, generator=g).to(DEV).requires_grad_()
+    leaves = [x, proj, a, bias]
+
+    def run():
+        out = selective_scan_gated(x, proj[..., :d], a, proj[..., d:d + n], proj[..., d + n:],
+                                   0.001, 0.1, return_state=True, dt_bias=bias)
+        return _grads(out, leaves, 2)
+    _compare(*_both(run), False)
