@@ -179,13 +179,20 @@ Segments segments_for(int64_t batch, int64_t D, int nch, int per_cu, bool carrie
 }
 
 // Plan shape of d_state N: states per lane and waves per block (false: none).
-bool plan_shape(int N, int& npl, int& G) {
+// dense_bwd: the gradient pass of a grid of at least a block per CU.
+bool plan_shape(int N, int& npl, int& G, bool dense_bwd = false) {
   if (N < 1 || N > MHS_MAX_DSTATE) return false;
   const int forced = g_npl_override.load(std::memory_order_relaxed);
   // Automatic: two states per lane up to d_state 32 (more, thinner blocks),
-  // four beyond. One state per lane: the instantiated plans pad d_state to 8
-  // or 16.
-  npl = forced != 0 ? forced : N <= 32 ? 2 : 4;
+  // four beyond. The gradient pass of a dense grid takes four from 17 on: a
+  // block of two states per lane there has 5 to 8 waves at three per SIMD,
+  // one block per CU whose barriers nothing covers, with four states 3 or 4
+  // waves and two blocks. Backward us, two / four states per lane:
+  // 16x512x1536 at d_state 18, 24, 32: 279 / 265, 294 / 272, 337 / 292;
+  // 8x1000x1000x32 (256 blocks) 264 / 242, 64x300x1024x32 529 / 427; sparser,
+  // 4x512x1536x32 (192 blocks) 107 / 125. (Forward: mixed, 117 / 99 and 178 /
+  // 202.) One state per lane: the instantiated plans pad d_state to 8 or 16.
+  npl = forced != 0 ? forced : N <= (dense_bwd ? 16 : 32) ? 2 : 4;
   G = npl == 1 ? (N <= 8 ? 4 : N <= 16 ? 8 : 0) : (N + 2 * npl - 1) / (2 * npl);
   return G >= 1 && G <= kMaxG;
 }
@@ -207,28 +214,37 @@ struct PassRate {
 // The split of a grid that leaves CUs without a block: segments and carry
 // units whose estimated time is the least (their walks, the carry pass, and
 // the fold of the units' carries at each segment's start, 0.2 us a unit,
-// more with several blocks per CU). The rates are those of MI355X at d_state
-// 16 and 64; the estimate was within 10% of the time of 200 measured splits
-// (2 to 210 blocks of 8 to 472 chunks) and its least within 2% of the
-// fastest on average (10% at worst). Against a limit of 8 segments of at
-// least 8 chunks, forward / backward us (GPU time):
-//   1x6664x64x16     109 -> 34 / 199 -> 44     1x1365x64x16  30 -> 20 / 48 -> 24
-//   2x7550x168x16     92 -> 47 / 162 -> 73     1x509x856x16  21 -> 18 / 32 -> 27
-//   4x1024x1024x64   136 -> 109 / 281 -> 216   3x1299x1924x64 266 -> 182 / 483 -> 445
-//   10x5749x666x16  (291) / 610 -> 505         3x1001x1432x16 bf16 (47) / 95 -> 76
+// more with several blocks per CU). The estimate is within 9% (rms) of 3,000
+// measured splits on MI355X (12 to 500 blocks of 25 to 188 chunks) and its
+// least within 3% of the fastest of them on average. Against a limit of 8
+// segments of at least 8 chunks, forward / backward us (GPU time; over 212
+// grids 23% / 17% faster on average):
+//   1x6664x64x16     120 -> 34 / 201 -> 42     1x1365x64x16   33 -> 20 / 49 -> 24
+//   2x7550x168x16    109 -> 52 / 166 -> 83     1x509x856x16   24 -> 19 / 33 -> 27
+//   4x1024x1024x64   146 -> 117 / 290 -> 231   3x1299x1924x64 277 -> 195 / 476 -> 447
+//   10x5749x666x16     (300) / 592 -> 532      8x2500x800x4   78 -> 66 / (135)
+//   10x700x740x32     94 -> 74 / 204 -> 150    3x2000x343x4   36 -> 26 / 61 -> 35
 constexpr int kMaxAutoSegments = 64, kMaxAutoUnits = 128;
 
 Segments least_segments(int64_t blocks, int nch, int cus, int npl, int G, bool fwd,
                         double unit_bytes) {
-  const double w = G * npl / 8.0;   // a block's VALU work against d_state 16's
-  const bool two = npl <= 2;
+  // us per chunk, fitted to the times of 19 grids at 12 d_states split 1 to 8
+  // ways. Up to four waves a block has a wave per SIMD, beyond that two.
+  const bool two = npl <= 2, thin = two && G <= 4;
   PassRate main, carry;
   if (fwd) {
-    main = {two ? std::max(1, 16 / G) : 1, two ? 0.97 : 2.2, 0.5 * w, 3.5};
-    carry = {two ? std::max(1, 20 / G) : 1, two ? 0.62 : 1.4, 0.3 * w, 3.5};
+    main = {std::max(1, (two ? 16 : 8) / G),
+            thin ? 0.8 + 0.05 * G : two ? 1 + 0.045 * G : 1.6 + 0.09 * G,
+            thin ? 0.1 + 0.06 * G : two ? (G == 5 ? 0.5 : 0.77) : 0.8 + 0.045 * G, 3.5};
+    carry = {std::max(1, (two ? 20 : 8) / G), thin ? 0.3 : two ? 1 : 1.2 + 0.06 * G,
+             thin ? 0.25 + 0.08 * G : two ? 0.2 + 0.08 * G : 0.6 + 0.03 * G, 3.5};
   } else {
-    main = {two ? std::max(1, 12 / G) : 1, two ? 2.1 : 5.3, 1.08 * w, 4.5};
-    carry = {two ? std::max(1, 16 / G) : 2, two ? 0.75 : 1.6, 0.33 * w, 4.5};
+    main = {std::max(1, (two ? 12 : 8) / G),
+            thin ? 2 + 0.02 * G : two ? 2.1 + 0.1 * G : 4 + 0.13 * G,
+            thin ? 0.42 + 0.14 * G : two ? 1.8 + 0.135 * G : 2.4, two ? 4.5 : 10};
+    carry = {std::max(1, 16 / G), thin ? 0.6 : two ? 0.22 * G - 0.4 : 0.3 + 0.4 * G,
+             thin ? 0.23 + 0.09 * G : two ? 0.7 : std::max(0.2, 0.25 * G - 0.26),
+             two ? 4.5 : 10};
   }
   const double launch = fwd ? 3 : 6;   // the carry pass's, and the zero fill's
   Segments best;
@@ -265,17 +281,29 @@ Segments least_segments(int64_t blocks, int nch, int cus, int npl, int G, bool f
 }
 
 // least_segments for a pass over (batch, D, N), or nothing where the split by
-// blocks per CU (segments_for) stands: forced splits, grids of a block per CU
-// or more, and forwards of up to 32 states from a quarter of that on (there
-// the two were within 4%). The last answers are kept per thread: the search
-// takes about 2 us, and a call asks up to three times.
+// blocks per CU (segments_for) stands: forced splits and dense grids. Blocks
+// of more than four waves, and of four states per lane, are estimated up to
+// two per CU: fewer of them share a CU than segments_for plans for, and one
+// segment is often the best (8x1000x1000x64, 256 blocks, forward / backward
+// 217 / 446 -> 158 / 369 us; 15x700x1000x64, 480 blocks, 316 / 593 -> 215 /
+// 497; 12x2000x1000x64, 384 blocks, 598 / 1167 -> 585 / 1151). Thinner blocks: the
+// line lies where the estimate's choice stops being the faster one on average:
+// forwards at four blocks to five CUs (of 65 to 200 blocks 11% faster, of 224
+// and 240 5% slower), of four waves at a quarter (at 48 to 250 within 4% on
+// average), gradients of four waves at a block per CU (3% faster up to there)
+// and of fewer waves at half of that (at 65 to 128 blocks 6% faster, at 143
+// to 250 1% slower and up to 12%). The last answers are kept per thread: the
+// search takes about 2 us, and a call asks up to three times.
 bool sparse_segments(int64_t batch, int64_t D, int64_t N, int nch, bool fwd, Segments& out) {
   if (g_seg_override.load(std::memory_order_relaxed) != 0) return false;
   const int64_t blocks = batch * ((D + mhs::kCH - 1) / mhs::kCH);
   const int cus = device_cus();
   int npl = 0, G = 0;
-  if (blocks >= cus || !plan_shape((int)N, npl, G)) return false;
-  if (fwd && npl <= 2 && 4 * blocks >= cus) return false;
+  if (!plan_shape((int)N, npl, G, !fwd && blocks >= cus)) return false;
+  if (npl == 4 || G > 4 ? blocks >= 2 * (int64_t)cus
+                        : fwd ? (G == 4 ? 4 * blocks >= cus : 5 * blocks > 4 * (int64_t)cus)
+                              : blocks >= (G == 4 ? cus : cus / 2 + 1))
+    return false;
   struct Entry { int64_t batch, D; int N, nch, cus, npl; bool fwd; Segments s; };
   thread_local Entry memo[8] = {};
   thread_local int next = 0;
@@ -405,9 +433,9 @@ bool fill_g1(int G, Plan& p) {
 }
 
 // Resolve the kernel variant for d_state N. Returns false if unsupported.
-bool make_plan(int N, Plan& p) {
+bool make_plan(int N, Plan& p, bool dense_bwd = false) {
   int npl = 0, G = 0;
-  if (!plan_shape(N, npl, G)) return false;
+  if (!plan_shape(N, npl, G, dense_bwd)) return false;
   const bool ok = npl == 2 ? fill_g<2>(G, p) : npl == 4 ? fill_g<4>(G, p)
                   : npl == 1 ? fill_g1(G, p) : false;
   if (!ok) return false;
@@ -798,9 +826,15 @@ int scan_bwd(const void* x, const void* dt, const float* aneg, const void* B, co
     if (q && !aligned16(q)) return fail(MHS_EINVAL, "device pointers must be 16-byte aligned");
   if (reinterpret_cast<uintptr_t>(workspace) & 255u)
     return fail(MHS_EINVAL, "workspace must be 256-byte aligned");
-  Plan p;
-  if (!make_plan((int)d_state, p)) return fail(MHS_EINVAL, "d_state %lld unsupported", (long long)d_state);
   const int ch = mhs::kCH;
+  // pf: the checkpoint recompute's plan, p: the adjoint's passes'.
+  Plan pf, p;
+  // (The gated swept kernel spills at four states per lane: 473 -> 506 us at
+  // 16x512x1536x32, stride 32.)
+  const bool dense = batch * ((d_inner + ch - 1) / ch) >= device_cus() &&
+                     !(g.on && sweep_km(chunk, seqlen, mhs::kSteps) > 0);
+  if (!make_plan((int)d_state, pf) || !make_plan((int)d_state, p, dense))
+    return fail(MHS_EINVAL, "d_state %lld unsupported", (long long)d_state);
   const WsLayout w = ws_layout(batch, seqlen, d_inner, d_state, chunk, p.bwd_ki);
   if (workspace_bytes < w.total)
     return fail(MHS_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, w.total);
@@ -839,7 +873,7 @@ int scan_bwd(const void* x, const void* dt, const float* aneg, const void* B, co
     f.h_init = ckpt;
     f.init_K = K;
     f.init_nchunk = (int)mhs_num_chunks(T, K);
-    rc = launch_fwd(p, f, (int)batch, s, g, e, nseg, /*ckpt_only=*/true);
+    rc = launch_fwd(pf, f, (int)batch, s, g, e, nseg, /*ckpt_only=*/true);
     if (rc) return rc;
     ck = f.ckpt;
     Kb = p.bwd_ki;

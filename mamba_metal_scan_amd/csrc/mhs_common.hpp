@@ -538,28 +538,36 @@ __device__ __forceinline__ void load_states(float (&v)[NPL], const GBuf& g, unsi
 // h <- carry_u + exp2(sdt_u * a2) h over the carry units u = first, first +
 // dir, ... (n of them) of the time segments: carry (unit, batch, slice) and
 // sdt (unit, batch, D) of this lane's states and channel. The loads of kFold
-// units are in flight together (one at a time, each unit costs a load's
-// latency, about a chunk's walk); units past n read as the identity (0, 0).
-constexpr int kFold = 8;
+// units are in flight together: one at a time, as the rest is, each unit
+// costs a load's latency, about a chunk's walk.
+constexpr int kFold = 4;
 template <int NPL>
 __device__ __forceinline__ void fold_carries(float (&h)[NPL], const float (&a2)[NPL],
                                              const float* carry, const float* sdt, int first,
                                              int dir, int n, int batch, int b, size_t slice,
                                              unsigned off, int nvalid, int sw, int D, int d) {
-  for (int u0 = 0; u0 < n; u0 += kFold) {
+  const auto load = [&](int u, float (&hv)[NPL], float& sd) {
+    const size_t slot = (size_t)(first + dir * u) * batch + b;
+    load_states<NPL>(hv, GBuf(carry + slot * slice, 4u * (unsigned)slice), off, nvalid, sw);
+    sd = GBuf(sdt + slot * D, 4u * (unsigned)D).ld(4u * (unsigned)d);
+  };
+  const auto fold = [&](const float (&hv)[NPL], float sd) {
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) h[j] = __builtin_fmaf(exp2_hw(sd * a2[j]), h[j], hv[j]);
+  };
+  int u0 = 0;
+  for (; u0 + kFold <= n; u0 += kFold) {
     float hv[kFold][NPL], sd[kFold];
 #pragma unroll
-    for (int i = 0; i < kFold; ++i) {
-      const bool in = u0 + i < n;
-      const size_t slot = (size_t)(first + dir * (in ? u0 + i : 0)) * batch + b;
-      load_states<NPL>(hv[i], GBuf(carry + slot * slice, in ? 4u * (unsigned)slice : 0u), off,
-                       nvalid, sw);
-      sd[i] = GBuf(sdt + slot * D, in ? 4u * (unsigned)D : 0u).ld(4u * (unsigned)d);
-    }
+    for (int i = 0; i < kFold; ++i) load(u0 + i, hv[i], sd[i]);
 #pragma unroll
-    for (int i = 0; i < kFold; ++i)
-#pragma unroll
-      for (int j = 0; j < NPL; ++j) h[j] = __builtin_fmaf(exp2_hw(sd[i] * a2[j]), h[j], hv[i][j]);
+    for (int i = 0; i < kFold; ++i) fold(hv[i], sd[i]);
+  }
+#pragma unroll 1
+  for (; u0 < n; ++u0) {
+    float hv[NPL], sd;
+    load(u0, hv, sd);
+    fold(hv, sd);
   }
 }
 

@@ -87,3 +87,48 @@ def test_gated_scan_in_many_segments():
                                    0.001, 0.1, return_state=True, dt_bias=bias)
         return _grads(out, leaves, 2)
     _compare(*_both(run), False)
+
+
+@pytest.mark.parametrize("bt,t,d,n,chunk", [
+    (6, 500, 1100, 4, 16), (5, 700, 1000, 12, 100), (7, 333, 1000, 16, 32), (7, 400, 1000, 24, 16),
+    (10, 300, 1000, 40, 64), (13, 250, 1200, 64, 16), (13, 250, 1200, 20, 48)])
+def test_middle_grids_equal_one_segment(bt, t, d, n, chunk):
+    """From two fifths of a block per CU to just under two, at each plan."""
+    print(f"[case] middle {bt}x{t}x{d}x{n} chunk {chunk}", flush=True)
+    g = torch.Generator().manual_seed(t + d + n)
+
+    def rand(*s):
+        return torch.randn(*s, generator=g).to(DEV)
+    leaves = [v.requires_grad_() for v in (rand(bt, t, d), F.softplus(rand(bt, t, d) - 4),
+                                           rand(d, n).abs(), rand(bt, t, n), rand(bt, t, n))]
+    auto, one = _both(lambda: _grads(
+        selective_scan_hip(*leaves, chunk=chunk, return_state=True), leaves, 1))
+    _compare(auto, one, False)
+
+
+@pytest.mark.parametrize("n,chunk,gated", [(17, 16, False), (24, 32, False), (25, 64, True),
+                                           (32, 16, True), (32, 32, True), (32, 48, False)])
+def test_dense_gradients_of_middle_states_equal_two_states_per_lane(n, chunk, gated):
+    """d_state 17..32 on a grid of a block per CU or more: four states per lane
+    in the gradient pass against two in every pass."""
+    bt, t, d = 8, 100, 1000 + 4 * (n % 2)
+    print(f"[case] dense {bt}x{t}x{d}x{n} chunk {chunk} gated {gated}", flush=True)
+    assert bt * ((d + 31) // 32) >= _native.library().mhs_cu_count()
+    g = torch.Generator().manual_seed(n + chunk)
+
+    def rand(*s):
+        return torch.randn(*s, generator=g).to(DEV)
+    leaves = [v.requires_grad_() for v in (rand(bt, t, d), F.softplus(rand(bt, t, d) - 4),
+                                           rand(d, n).abs(), rand(bt, t, n), rand(bt, t, n))]
+
+    def run():
+        out = (selective_scan_gated(*leaves, 0.001, 0.1, chunk=chunk, return_state=True) if gated
+               else selective_scan_hip(*leaves, chunk=chunk, return_state=True))
+        return _grads(out, leaves, 1)
+    auto = run()
+    _native.set_variant(2)
+    try:
+        two = run()
+    finally:
+        _native.set_variant(0)
+    _compare(auto, two, False)
