@@ -673,6 +673,7 @@ def pmc_summary(args) -> None:
 
 
 TRAIN_GROUPS = (  # (label, substrings of the kernel name), first match wins
+    ("HIP fp32 GEMMs (three bf16 parts)", ("mhs::gemm", "mhs::concat3")),
     ("fp32 GEMMs (rocBLAS / hipBLASLt)", ("Cijk_", "gemm", "Gemm")),
     ("HIP scan (fwd, bwd, reduce)", ("mhs::fwd_kernel", "mhs::bwd_kernel", "mhs::bwd_reduce")),
     ("HIP conv1d + SiLU", ("mhs::conv",)),

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from helpers import assert_close
-from mamba_metal_scan_amd import block as block_mod
+from mamba_metal_scan_amd import _native, block as block_mod
 from mamba_metal_scan_amd.model import MambaBlock, MambaConfig, TinyMamba
 
 pytestmark = pytest.mark.gpu
@@ -156,3 +156,35 @@ def test_model_gradients_equal_the_module_path():
     assert_close("loss", loss, loss2, tol=1e-6)
     for k in native:
         assert_close(k, native[k], module[k], tol=2e-5)
+
+
+def test_forward_and_gradients_replay_from_a_hip_graph():
+    """The native block's launches captured once and replayed three times, with
+    eager work between: every replay equals the eager result."""
+    hip, _ = _blocks(64, 96)
+    g = torch.Generator().manual_seed(4)
+    x = torch.randn(2, 65, 64, generator=g).to(DEV).requires_grad_()
+    dy = torch.randn(2, 65, 64, generator=g).to(DEV)
+    leaves = [x] + list(hip.parameters())
+
+    def step(inputs):
+        out = hip(inputs[0])
+        return (out,) + torch.autograd.grad(out, inputs, dy)
+    _native.set_reduction(_native.REDUCTION_FIXED)
+    try:
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            ref = [v.detach().clone() for v in step(leaves)]
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            outs = step(leaves)
+        for rep in range(3):
+            torch.randn(1 << 20, device=DEV).sum().item()   # eager work between replays
+            graph.replay()
+            torch.cuda.synchronize()
+            for i, (a, b) in enumerate(zip(outs, ref)):
+                assert torch.equal(a, b), f"replay {rep}: output {i} differs"
+    finally:
+        _native.set_reduction(_native.REDUCTION_AUTO)

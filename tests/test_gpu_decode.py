@@ -121,3 +121,41 @@ def test_windows_of_earlier_steps_are_kept():
         first, _ = hip(idx[:, 7:8], cache=cache)
         again, _ = hip(idx[:, 7:8], cache=snap)
     assert torch.equal(first, again)
+
+
+def test_token_replays_from_a_hip_graph():
+    """One captured token (the cache it reads written back in place between
+    replays): three replays, with eager work between, equal the eager token."""
+    hip, _ = _models()
+    idx = torch.randint(0, hip.cfg.vocab_size, (2, 7), generator=torch.Generator().manual_seed(2))
+    idx = idx.to(DEV)
+    with torch.no_grad():
+        cache = {}
+        hip(idx[:, :6], cache=cache)
+        saved = [{k: v.clone() for k, v in b.items()} for b in cache["blocks"]]
+
+        def token():
+            c = {"blocks": [dict(b) for b in start]}
+            return hip(idx[:, 6:], cache=c)[0]
+        start = [{k: v.clone() for k, v in b.items()} for b in saved]
+
+        def restore():
+            for b, s in zip(start, saved):
+                for k in s:
+                    b[k].copy_(s[k])
+        ref = token().clone()
+        restore()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            token()
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = token()
+        for rep in range(3):
+            restore()
+            torch.randn(1 << 20, device=DEV).sum().item()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, ref), f"replay {rep}"
