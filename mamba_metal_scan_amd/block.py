@@ -28,10 +28,11 @@ def plain(t: Optional[torch.Tensor], dev: torch.device, shape: tuple) -> bool:
 
 
 def plain_mods(mods, kinds) -> bool:
-    """Whether each module is of exactly its kind, without hooks of its own."""
+    """Whether each module is of exactly its kind, without hooks or a forward
+    of its own."""
     for mod, kind in zip(mods, kinds):
         if (type(mod) is not kind or mod._forward_hooks or mod._forward_pre_hooks
-                or mod._backward_hooks or mod._backward_pre_hooks):
+                or mod._backward_hooks or mod._backward_pre_hooks or "forward" in mod.__dict__):
             return False
     return True
 
@@ -39,7 +40,8 @@ def plain_mods(mods, kinds) -> bool:
 def block_params(block: nn.Module, x: torch.Tensor, strict: bool) -> Optional[tuple]:
     """The block's parameters in mhs_block_weights' order where the native
     block takes them and x (batch, T, d_model), else None: plain modules
-    without hooks (strict: those too that the block's fused path never calls),
+    without hooks or a forward of their own (strict: those too that the
+    block's fused path never calls),
     fp32 contiguous 16-byte aligned parameters of the block's shapes, sizes
     that are multiples of 4. The caller has checked the global hooks,
     autocast, tracing and that x is an fp32 ROCm tensor."""

@@ -29,8 +29,8 @@ _f32 = torch.float32
 def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: tuple,
            conv_next: torch.Tensor) -> Optional[bytes]:
     """The block's mhs_decode_layer, or None where the native step does not
-    take it: a module of another type or with hooks, a weight that is not a
-    plain fp32 parameter of its shape, a state or window that is not the
+    take it: a module of another type, with hooks or with a forward of its
+    own, a weight that is not a plain fp32 parameter of its shape, a state or window that is not the
     cache's own form."""
     m, p = block._modules, block._parameters
     try:
@@ -68,8 +68,8 @@ def decode_step(model: nn.Module, x: torch.Tensor, cache: dict) -> Optional[torc
     """The logits (batch, 1, vocab) of one embedded token per sequence, x
     (batch, 1, d_model), against a filled cache, which is advanced (each
     block's h in place, its conv window replaced). None (and nothing changed)
-    where the native step does not apply: modules with hooks or of other
-    types, other dtypes or layouts, autocast, or a cache that no prefill
+    where the native step does not apply: modules with hooks, with a forward
+    set on the instance or of other types, other dtypes or layouts, autocast, or a cache that no prefill
     filled. The caller has checked that autograd is off and that every block
     is a plain MambaBlock."""
     blocks, states, head, ln_f = model.blocks, cache["blocks"], model.head, model.ln_f

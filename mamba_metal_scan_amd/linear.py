@@ -37,18 +37,20 @@ class LinearHIP(torch.autograd.Function):
 
 
 def no_hooks(m: nn.Module) -> bool:
-    """Whether neither m nor the module-global registries hold forward or
-    backward hooks."""
+    """Whether calling m runs its class's forward alone: neither m nor the
+    module-global registries hold forward or backward hooks, and m has no
+    forward of its own (set on the instance, as adapters, offloading and
+    instrumentation do)."""
     g = nn.modules.module
     return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                or m._backward_pre_hooks or g._global_forward_hooks
+                or m._backward_pre_hooks or "forward" in m.__dict__ or g._global_forward_hooks
                 or g._global_forward_pre_hooks or g._global_backward_hooks
                 or g._global_backward_pre_hooks)
 
 
 def linear(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """mod(x), through the HIP products where mod is a plain bias-free
-    nn.Linear (no subclass, no hooks), x and its weight are fp32 on one ROCm
+    nn.Linear (no subclass, no hooks, no forward of its own), x and its weight are fp32 on one ROCm
     device outside autocast, and the product is large enough to be the faster
     there (smaller ones keep the framework's call and its lower overhead)."""
     if (type(mod) is nn.Linear and mod.bias is None and x.is_cuda and x.dtype == torch.float32

@@ -305,7 +305,7 @@ class MambaBlock(nn.Module):
         read directly, as in the fused path). With a cache (a prefill, without
         autograd) it is filled."""
         norm = self._modules["norm"]
-        if (type(self) is not MambaBlock or self.scan_impl == "torch" or type(norm) is not RMSNorm
+        if (not _own_methods(self) or self.scan_impl == "torch" or type(norm) is not RMSNorm
                 or not norm.uses_hip(x) or x.dim() != 3 or not no_hooks(norm)
                 or torch.is_autocast_enabled() or torch.compiler.is_compiling()):
             return None
@@ -334,7 +334,7 @@ class MambaBlock(nn.Module):
         r = self._native(x, None, cache)
         if r is not None:
             return r[0] + r[1]
-        if self.norm.uses_hip(x):
+        if self.norm.uses_hip(x) and no_hooks(self.norm):
             # x itself, and its norm; the backward adds x's two gradients in
             # the norm's kernel.
             residual, h = rms_norm_residual(x, self.norm.weight, self.norm.eps)
@@ -369,11 +369,20 @@ class MambaBlock(nn.Module):
         return self.out_proj(y * F.silu(z))
 
 
+_METHODS = tuple(k for k, v in vars(MambaBlock).items() if callable(v) and k != "__init__")
+
+
+def _own_methods(b: nn.Module) -> bool:
+    """Whether b is a MambaBlock itself (not a wrapper or a subclass) that runs
+    the class's methods, none of them set on the instance."""
+    return type(b) is MambaBlock and not any(k in b.__dict__ for k in _METHODS)
+
+
 def _plain_block(b: nn.Module) -> bool:
-    """Whether calling b.mix() in place of b(x) skips nothing: b is a
-    MambaBlock itself (not a wrapper or a subclass) and neither it nor the
-    module-global registries hold forward or backward hooks."""
-    return type(b) is MambaBlock and no_hooks(b)
+    """Whether calling b.mix() in place of b(x) skips nothing: b runs the
+    class's own methods, and neither b, its norm nor the module-global
+    registries hold forward or backward hooks."""
+    return _own_methods(b) and no_hooks(b) and no_hooks(b.norm)
 
 
 class TinyMamba(nn.Module):
@@ -406,8 +415,8 @@ class TinyMamba(nn.Module):
 
     def _hidden(self, x, caches):
         """The final norm's output for the embedded tokens x."""
-        if self.ln_f.uses_hip(x) and all(_plain_block(b) and b.norm.uses_hip(x)
-                                         for b in self.blocks):
+        if (self.ln_f.uses_hip(x) and no_hooks(self.ln_f)
+                and all(_plain_block(b) and b.norm.uses_hip(x) for b in self.blocks)):
             # The HIP norms: each block's residual add goes into the next norm's
             # kernel (x + delta and its norm in one pass). This calls each
             # block's mix() rather than the block itself, so it is taken only

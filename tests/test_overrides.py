@@ -1,0 +1,148 @@
+"""Modules whose forward (or, of a block, any method) is set on the instance,
+as adapters, offloading and instrumentation do, and weights that are not plain
+tensors: every path of the model that calls such a module runs its override,
+and the native paths refuse it.
+"""
+from __future__ import annotations
+
+import copy
+
+import pytest
+import torch
+import torch.nn as nn
+
+from helpers import assert_close
+from mamba_metal_scan_amd.block import plain_mods
+from mamba_metal_scan_amd.linear import no_hooks
+from mamba_metal_scan_amd.model import MambaBlock, MambaConfig, TinyMamba, _plain_block
+
+DEV = "cuda"
+
+
+def _model(vocab=203):
+    torch.manual_seed(2)
+    m = TinyMamba(MambaConfig(vocab_size=vocab, d_model=64, n_layers=2, d_ff=128,
+                              scan_impl="hip"))
+    with torch.no_grad():
+        for b in m.blocks:
+            b.dt_proj.bias.normal_()
+            b.conv.bias.normal_()
+    return m
+
+
+# -------------------------------------------------------- the predicates (CPU)
+
+def test_an_overridden_forward_is_not_plain():
+    lin = nn.Linear(4, 4, bias=False)
+    assert plain_mods((lin,), (nn.Linear,)) and no_hooks(lin)
+    lin.forward = lambda x: x
+    assert not plain_mods((lin,), (nn.Linear,)) and not no_hooks(lin)
+    del lin.forward
+    assert plain_mods((lin,), (nn.Linear,)) and no_hooks(lin)
+
+
+@pytest.mark.parametrize("where", ["forward", "mix", "_step", "_scan", "norm.forward"])
+def test_a_block_with_a_method_of_its_own_is_not_plain(where):
+    block = _model().blocks[0]
+    assert _plain_block(block)
+    owner = block.norm if where.startswith("norm") else block
+    setattr(owner, where.split(".")[-1], lambda *a, **k: None)
+    assert not _plain_block(block)
+
+
+# ------------------------------------------------------------- every path (GPU)
+
+def _run(m, path, idx):
+    """(logits, cache tensors) of one path over the tokens idx."""
+    if path == "train":
+        return (m(idx)[0],)
+    with torch.no_grad():
+        cache = {}
+        logits = m(idx[:, :-1] if path == "token" else idx, cache=cache)[0]
+        if path == "token":
+            logits = m(idx[:, -1:], cache=cache)[0]
+    return (logits, *[b[k] for b in cache["blocks"] for k in ("h", "conv")])
+
+
+def _double(mod):
+    """mod's forward set on the instance: twice the class's."""
+    calls = []
+
+    def forward(*args):
+        calls.append(1)
+        return 2 * type(mod).forward(mod, *args)
+    mod.forward = forward
+    return calls
+
+
+# Training calls in_proj, out_proj and the head as modules, a prompt and a
+# token the other projections too, a token the conv.
+@pytest.mark.gpu
+@pytest.mark.parametrize("path,name", [
+    (p, n) for p, ns in (("train", "in_proj out_proj"),
+                         ("prefill", "in_proj out_proj dt_proj B_proj C_proj"),
+                         ("token", "in_proj out_proj dt_proj B_proj C_proj conv"))
+    for n in ns.split()])
+def test_child_forward_runs(path, name):
+    print(f"[case] override {path} {name}", flush=True)
+    m = _model().to(DEV)
+    idx = torch.randint(0, 203, (3, 9), generator=torch.Generator().manual_seed(1)).to(DEV)
+    want = copy.deepcopy(m)
+    with torch.no_grad():
+        for p in getattr(want.blocks[1], name).parameters():
+            p.mul_(2)
+    if path == "token":   # alone: both caches from the plain model's prompt
+        plain = {}
+        with torch.no_grad():
+            m(idx[:, :-1], cache=plain)
+
+        def step(model):
+            cache = {"blocks": [{k: v.clone() for k, v in b.items()} for b in plain["blocks"]]}
+            with torch.no_grad():
+                logits = model(idx[:, -1:], cache=cache)[0]
+            return (logits, *[b[k] for b in cache["blocks"] for k in ("h", "conv")])
+        ref = step(want)
+        calls = _double(getattr(m.blocks[1], name))
+        got = step(m)
+    else:
+        ref = _run(want, path, idx)
+        calls = _double(getattr(m.blocks[1], name))
+        got = _run(m, path, idx)
+    torch.cuda.synchronize()
+    assert calls == [1]
+    for i, (a, b) in enumerate(zip(got, ref)):
+        assert_close(f"output {i}", a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["train", "prefill", "token"])
+def test_head_and_norm_forward_run(path):
+    """The head at a size the HIP product would take (512 x 32768 x 64)."""
+    print(f"[case] override head, norms {path}", flush=True)
+    m = _model(vocab=32768).to(DEV)
+    idx = torch.randint(0, 32768, (4, 128), generator=torch.Generator().manual_seed(1)).to(DEV)
+    m.head.forward = lambda x: x.sum(-1, keepdim=True)
+    calls = [_double(mod) for mod in (m.ln_f, m.blocks[0].norm)]
+    logits = _run(m, path, idx)[0]
+    assert logits.shape == (4, 1 if path == "token" else 128, 1)
+    n = 2 if path == "token" else 1
+    assert [len(c) for c in calls] == [n, n]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["train", "prefill", "token"])
+@pytest.mark.parametrize("method", ["forward", "mix"])
+def test_block_method_runs(path, method):
+    print(f"[case] override block {method} {path}", flush=True)
+    m = _model().to(DEV)
+    idx = torch.randint(0, 203, (2, 9), generator=torch.Generator().manual_seed(1)).to(DEV)
+    want = _run(m, path, idx)
+    block, calls = m.blocks[0], []
+
+    def own(*args):
+        calls.append(1)
+        return getattr(MambaBlock, method)(block, *args)
+    setattr(block, method, own)
+    for i, (a, b) in enumerate(zip(_run(m, path, idx), want)):
+        assert_close(f"output {i}", a, b)
+    assert len(calls) == (2 if path == "token" else 1)
