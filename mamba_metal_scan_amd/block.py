@@ -15,6 +15,7 @@ import torch
 import torch.nn as nn
 
 from . import _native
+from .linear import PLAIN
 
 _WEIGHTS = struct.Struct("11Q4f")      # mhs_block_weights
 _GRADS = struct.Struct("10Q")          # mhs_block_grads
@@ -22,8 +23,8 @@ _f32 = torch.float32
 
 
 def plain(t: Optional[torch.Tensor], dev: torch.device, shape: tuple) -> bool:
-    """Whether t is fp32 of that shape, contiguous, on dev."""
-    return (t is not None and t.dtype is _f32 and t.shape == shape and t.device == dev
+    """Whether t is a plain tensor, fp32 of that shape, contiguous, on dev."""
+    return (type(t) in PLAIN and t.dtype is _f32 and t.shape == shape and t.device == dev
             and t.is_contiguous())
 
 

@@ -16,7 +16,7 @@ import torch.nn as nn
 
 from . import _native
 from .block import plain, plain_mods
-from .linear import no_hooks
+from .linear import PLAIN, no_hooks
 
 # mhs_decode_layer: 13 pointers, the conv window's strides, the next window,
 # eps, dt_min, dt_max, unused.
@@ -52,7 +52,7 @@ def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: 
     for t, shape in zip(weights, shapes):
         if not plain(t, dev, shape):
             return None
-    if (any(v is not None for v in biases) or win is None or win.dtype is not _f32
+    if (any(v is not None for v in biases) or type(win) not in PLAIN or win.dtype is not _f32
             or win.shape != shapes[12] or win.device != dev or not norm.hip
             or block.scan_impl == "torch" or not block.dt_min < block.dt_max):
         return None
@@ -69,13 +69,14 @@ def decode_step(model: nn.Module, x: torch.Tensor, cache: dict) -> Optional[torc
     (batch, 1, d_model), against a filled cache, which is advanced (each
     block's h in place, its conv window replaced). None (and nothing changed)
     where the native step does not apply: modules with hooks, with a forward
-    set on the instance or of other types, other dtypes or layouts, autocast, or a cache that no prefill
-    filled. The caller has checked that autograd is off and that every block
-    is a plain MambaBlock."""
+    set on the instance or of other types, tensors of subclasses, other
+    dtypes or layouts, autocast, or a cache that no prefill filled. The
+    caller has checked that autograd is off and that every block is a plain
+    MambaBlock."""
     blocks, states, head, ln_f = model.blocks, cache["blocks"], model.head, model.ln_f
     if (torch.is_autocast_enabled() or torch.compiler.is_compiling() or x.dim() != 3
-            or x.dtype != torch.float32 or x.numel() == 0 or len(blocks) == 0
-            or len(states) != len(blocks)):
+            or type(x) not in PLAIN or x.dtype != torch.float32 or x.numel() == 0
+            or len(blocks) == 0 or len(states) != len(blocks)):
         return None
     first = blocks[0]
     if type(first.conv) is not nn.Conv1d or type(head) is not nn.Linear:

@@ -36,6 +36,11 @@ class LinearHIP(torch.autograd.Function):
         return dx, dw
 
 
+# A tensor of another type may have no storage of its own, or operators that
+# mean something else.
+PLAIN = (torch.Tensor, nn.Parameter)
+
+
 def no_hooks(m: nn.Module) -> bool:
     """Whether calling m runs its class's forward alone: neither m nor the
     module-global registries hold forward or backward hooks, and m has no
@@ -57,8 +62,9 @@ def linear(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
             and torch.version.hip is not None and not torch.is_autocast_enabled()):
         w = mod.weight
         k = x.shape[-1]
-        if (k > 0 and w.dtype == torch.float32 and w.device == x.device and w.shape[1] == k
-                and w.is_contiguous() and no_hooks(mod)
+        if (k > 0 and type(w) in PLAIN and type(x) in PLAIN and w.dtype == torch.float32
+                and w.device == x.device and w.shape[1] == k and w.is_contiguous()
+                and no_hooks(mod)
                 and _native.gemm_preferred(x.numel() // k, w.shape[0], k)):
             x2 = x.reshape(-1, k)
             return LinearHIP.apply(x2, w).view(*x.shape[:-1], w.shape[0])

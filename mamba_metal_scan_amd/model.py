@@ -42,7 +42,7 @@ from .block import BlockHIP, block_forward, block_params
 from .conv import conv1d_silu
 from .decode import decode_step
 from .fused import mamba_inner, out_gate, selective_scan_gated
-from .linear import linear, no_hooks
+from .linear import PLAIN, linear, no_hooks
 from .norm import add_rms_norm, rms_norm, rms_norm_residual
 from .scan import SSM_CHUNK, _hip_device, selective_scan, selective_state_step
 from .xent import cross_entropy
@@ -306,7 +306,8 @@ class MambaBlock(nn.Module):
         autograd) it is filled."""
         norm = self._modules["norm"]
         if (not _own_methods(self) or self.scan_impl == "torch" or type(norm) is not RMSNorm
-                or not norm.uses_hip(x) or x.dim() != 3 or not no_hooks(norm)
+                or type(x) not in PLAIN or not norm.uses_hip(x) or x.dim() != 3
+                or not no_hooks(norm)
                 or torch.is_autocast_enabled() or torch.compiler.is_compiling()):
             return None
         grad = torch.is_grad_enabled()
@@ -317,7 +318,8 @@ class MambaBlock(nn.Module):
             return None
         x = _aligned(x)
         if delta is not None:
-            if delta.shape != x.shape or delta.dtype != x.dtype or delta.device != x.device:
+            if (type(delta) not in PLAIN or delta.shape != x.shape or delta.dtype != x.dtype
+                    or delta.device != x.device):
                 return None
             delta = _aligned(delta)
         consts = (norm.eps, self.dt_min, self.dt_max, self.ckpt_chunk)

@@ -12,7 +12,7 @@ import torch
 import torch.nn as nn
 
 from helpers import assert_close
-from mamba_metal_scan_amd.block import plain_mods
+from mamba_metal_scan_amd.block import plain, plain_mods
 from mamba_metal_scan_amd.linear import no_hooks
 from mamba_metal_scan_amd.model import MambaBlock, MambaConfig, TinyMamba, _plain_block
 
@@ -48,6 +48,43 @@ def test_a_block_with_a_method_of_its_own_is_not_plain(where):
     owner = block.norm if where.startswith("norm") else block
     setattr(owner, where.split(".")[-1], lambda *a, **k: None)
     assert not _plain_block(block)
+
+
+class Doubled(torch.Tensor):
+    """A wrapper without storage of its own: twice the tensor it holds, as a
+    quantised weight inside a plain nn.Linear would be computed from its codes."""
+
+    @staticmethod
+    def __new__(cls, inner):
+        return torch.Tensor._make_wrapper_subclass(cls, inner.shape, dtype=inner.dtype,
+                                                   device=inner.device)
+
+    def __init__(self, inner):
+        self.inner = inner
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        if func is torch.ops.aten.detach.default:
+            return cls(args[0].inner)
+        args = torch.utils._pytree.tree_map_only(cls, lambda t: 2 * t.inner, args)
+        return func(*args, **(kwargs or {}))
+
+
+class Tagged(torch.Tensor):
+    """A subclass with storage, whose operators double their results."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        out = super().__torch_function__(func, types, args, kwargs)
+        return 2 * out.as_subclass(torch.Tensor) if func is torch.nn.functional.linear else out
+
+
+def test_a_subclass_is_not_plain():
+    t = torch.randn(4, 4)
+    assert plain(t, t.device, t.shape) and plain(nn.Parameter(t), t.device, t.shape)
+    assert not plain(Doubled(t), t.device, t.shape)
+    assert not plain(t.as_subclass(Tagged), t.device, t.shape)
+    assert not plain(None, t.device, t.shape)
 
 
 # ------------------------------------------------------------- every path (GPU)
@@ -146,3 +183,25 @@ def test_block_method_runs(path, method):
     for i, (a, b) in enumerate(zip(_run(m, path, idx), want)):
         assert_close(f"output {i}", a, b)
     assert len(calls) == (2 if path == "token" else 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["train", "prefill", "token"])
+@pytest.mark.parametrize("kind", [Doubled, Tagged])
+def test_subclassed_weights_keep_their_operators(path, kind):
+    """in_proj, out_proj and the head (512 x 32768 x 64: a size the HIP product
+    would take) with weights of a subclass that stands for twice its values."""
+    print(f"[case] subclassed weights {kind.__name__} {path}", flush=True)
+    m = _model(vocab=32768).to(DEV)
+    m.head.weight = nn.Parameter(m.head.weight.detach().clone())
+    idx = torch.randint(0, 32768, (4, 128), generator=torch.Generator().manual_seed(1)).to(DEV)
+    want = copy.deepcopy(m)
+    for model, double in ((want, lambda w: 2 * w),
+                          (m, lambda w: kind(w) if kind is Doubled else w.as_subclass(kind))):
+        for mod in (model.head, model.blocks[0].in_proj, model.blocks[1].out_proj):
+            w = double(mod.weight.detach())
+            mod.weight = nn.Parameter(w, requires_grad=False)
+            assert type(mod.weight) in (nn.Parameter, kind)
+    ref = _run(want, path, idx)
+    for i, (a, b) in enumerate(zip(_run(m, path, idx), ref)):
+        assert_close(f"output {i}", a.as_subclass(torch.Tensor), b)
