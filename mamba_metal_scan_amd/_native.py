@@ -1131,10 +1131,17 @@ def _gemm_sizes(a: torch.Tensor, b: torch.Tensor, form: int) -> tuple[int, int, 
     return m, b.shape[0] if form == GEMM_NT else b.shape[1], k
 
 
-@torch.compiler.assume_constant_result
+GEMM_LEAST = 1 << 30   # multiply-adds below which the framework's product is the faster
+
+
 def gemm_preferred(m: int, n: int, k: int) -> bool:
     """Whether the HIP product is the faster at these sizes (else the
-    framework's)."""
+    framework's). While torch.compile or torch.export traces, whether it may
+    be: sizes that are symbolic there are known at each call of the gemm op
+    only, whose implementation then chooses."""
+    if torch.compiler.is_compiling():
+        from torch.fx.experimental.symbolic_shapes import statically_known_true
+        return not statically_known_true(m * n * k < GEMM_LEAST)
     return library().mhs_gemm_preferred(m, n, k) != 0
 
 

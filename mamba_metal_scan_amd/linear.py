@@ -14,6 +14,7 @@ import torch.nn.functional as F
 
 from . import _native
 from ._native import GEMM_NN, GEMM_NT, GEMM_TN, dispatch
+from .scan import _hip_device
 
 
 class LinearHIP(torch.autograd.Function):
@@ -58,8 +59,8 @@ def linear(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
     nn.Linear (no subclass, no hooks, no forward of its own), x and its weight are fp32 on one ROCm
     device outside autocast, and the product is large enough to be the faster
     there (smaller ones keep the framework's call and its lower overhead)."""
-    if (type(mod) is nn.Linear and mod.bias is None and x.is_cuda and x.dtype == torch.float32
-            and torch.version.hip is not None and not torch.is_autocast_enabled()):
+    if (type(mod) is nn.Linear and mod.bias is None and _hip_device(x)
+            and x.dtype == torch.float32 and not torch.is_autocast_enabled()):
         w = mod.weight
         k = x.shape[-1]
         if (k > 0 and type(w) in PLAIN and type(x) in PLAIN and w.dtype == torch.float32

@@ -199,6 +199,29 @@ def test_compiled_tinymamba_train_step_matches_eager():
         assert_close(name, a, b, 1e-5)
 
 
+def test_compiled_tinymamba_at_changing_batches():
+    """One compiled TinyMamba at several batch sizes, the last of them with a
+    head (512 x 32768 x 64) large enough for the HIP product."""
+    from mamba_metal_scan_amd import MambaConfig, TinyMamba
+    print("[case] torch.compile TinyMamba, batches", flush=True)
+    torch.manual_seed(0)
+    model = TinyMamba(MambaConfig(vocab_size=32768, d_model=64, n_layers=2, d_ff=128,
+                                  max_seq_len=64, d_state=16, scan_impl="hip")).to(DEV)
+    fn = torch.compile(model, backend="aot_eager", fullgraph=True)
+    for batch in (2, 3, 16):
+        idx = torch.randint(0, 32768, (batch, 33), generator=_gen(batch)).to(DEV)
+        results = []
+        for f in (model, fn):
+            model.zero_grad(set_to_none=True)
+            logits, loss = f(idx[:, :-1], idx[:, 1:])
+            loss.backward()
+            results.append([logits.detach(), loss.detach()]
+                           + [p.grad.clone() for p in model.parameters()])
+        torch.cuda.synchronize()
+        for i, (a, b) in enumerate(zip(*results)):
+            assert_close(f"batch {batch}: {i}", a, b, 1e-5)
+
+
 def _capture(fn):
     """fn() warmed up on a side stream, then captured in a HIP graph; returns
     (graph, the captured outputs)."""
