@@ -64,14 +64,45 @@ def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: 
                        block.dt_min, block.dt_max, 0.0)
 
 
+def batch_limit(d_model: int, d_inner: int, d_state: int, n_layers: int, vocab: int,
+                captured: bool) -> int:
+    """The largest batch that the native token takes.
+
+    Its products pass over their weights, 512 columns at a time, again for
+    every 8 rows, with VALU fmas: a layer (with its share of the head) costs
+    0.45 us a row and 0.136 us a row and million of weights so padded. The
+    module calls reuse tiles in the library's products: about 0.25 us a row
+    and 0.055 us a row and million weights, but on top of the launches, about
+    300 us a layer from Python and 70 to 170 us in a HIP graph. The line lies
+    where the native rows have used that up, with a margin: measured us a
+    token, native / modules, at the last batch won and the first lost, and
+    the line (vocabulary 32768; 200 at d_model 1024),
+      d_model, d_inner, layers  from Python                                in a graph
+      128, 272, 2        128: 450 / 705    256: 868 / 703    168    24: 114 / 136     32: 143 / 142     31
+      384, 856, 10       256: 2711 / 3409  512: 5313 / 3262  287   192: 2016 / 2153  256: 2702 / 2405   73
+      640, 1432, 12      128: 2632 / 4045  256: 5008 / 4045  167    96: 2031 / 2276  128: 2617 / 2454   38
+      1024, 2312, 24      64: 4393 / 7596  128: 8205 / 7996  123    64: 4363 / 4943   96: 6252 / 5809   30
+      1536, 3472, 8       32: 1633 / 2573   64: 2921 / 2712   53    24: 1302 / 1406   32: 1635 / 1588   13
+    Up to 8 rows the weights are read once, as any product must."""
+    def padded(k: int) -> int:
+        return (k + 511) // 512 * 512
+    wide = 2 * d_inner * padded(d_model) + (d_inner + 2 * d_state + d_model) * padded(d_inner)
+    wide += vocab * padded(d_model) / n_layers
+    plain_w = d_inner * (3 * d_model + d_inner + 2 * d_state) + vocab * d_model / n_layers
+    native = 0.45 + 0.136e-6 * wide
+    rows = 41.0 / (native - 0.25 - 0.055e-6 * plain_w) if captured else 280.0 / native
+    return max(8, int(rows))
+
+
 def decode_step(model: nn.Module, x: torch.Tensor, cache: dict) -> Optional[torch.Tensor]:
     """The logits (batch, 1, vocab) of one embedded token per sequence, x
     (batch, 1, d_model), against a filled cache, which is advanced (each
     block's h in place, its conv window replaced). None (and nothing changed)
     where the native step does not apply: modules with hooks, with a forward
     set on the instance or of other types, tensors of subclasses, other
-    dtypes or layouts, autocast, or a cache that no prefill filled. The
-    caller has checked that autograd is off and that every block is a plain
+    dtypes or layouts, autocast, a cache that no prefill filled, or a batch
+    above batch_limit, where the modules are the faster. The caller has
+    checked that autograd is off and that every block is a plain
     MambaBlock."""
     blocks, states, head, ln_f = model.blocks, cache["blocks"], model.head, model.ln_f
     if (torch.is_autocast_enabled() or torch.compiler.is_compiling() or x.dim() != 3
@@ -87,7 +118,9 @@ def decode_step(model: nn.Module, x: torch.Tensor, cache: dict) -> Optional[torc
     x = x.contiguous()
     if (not no_hooks(head) or not no_hooks(ln_f) or type(ln_f) is not type(first.norm)
             or head.bias is not None or not ln_f.hip
-            or d_model % 4 or d % 4 or not 2 <= taps <= 8 or not 1 <= n <= 64 or batch > 65535):
+            or d_model % 4 or d % 4 or not 2 <= taps <= 8 or not 1 <= n <= 64
+            or batch > 8 and batch > batch_limit(d_model, d, n, len(blocks), head.out_features,
+                                                 torch.cuda.is_current_stream_capturing())):
         return None
     head_w, norm_w = head._parameters.get("weight"), ln_f._parameters.get("weight")
     if (not plain(norm_w, dev, (d_model,)) or not plain(head_w, dev, (head.out_features, d_model))

@@ -76,6 +76,36 @@ def test_token_matches_float64(monkeypatch, batch, over):
     assert seen == [True] * 3
 
 
+def test_batches_on_both_sides_of_the_limit(monkeypatch):
+    """The largest batch of the native token and the next, which takes the
+    module calls; both follow the float64 step."""
+    hip, ref = _models(n_layers=1)
+    limit = decode.batch_limit(64, hip.d_inner, 16, 1, 203, False)
+    assert 8 < limit < 1024
+    seen = _native_calls(monkeypatch)
+    for batch, native in ((limit, True), (limit + 1, False)):
+        idx = torch.randint(0, 203, (batch, 4), generator=torch.Generator().manual_seed(batch))
+        ch, cr = {}, {}
+        with torch.no_grad():
+            hip(idx[:, :3].to(DEV), cache=ch)
+            ref(idx[:, :3], cache=cr)
+            lh, _ = hip(idx[:, 3:].to(DEV), cache=ch)
+            lr, _ = ref(idx[:, 3:], cache=cr)
+        assert_close("logits", lh, lr)
+        assert_close("h", ch["blocks"][0]["h"], cr["blocks"][0]["h"])
+        assert seen.pop() is native
+    # in a HIP graph the modules' launches cost less: the line is lower
+    low = decode.batch_limit(64, hip.d_inner, 16, 1, 203, True)
+    assert 8 <= low < limit
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    for batch, native in ((low, True), (low + 1, False)):
+        cache, idx = {}, torch.zeros((batch, 2), dtype=torch.int64, device=DEV)
+        with torch.no_grad():
+            hip(idx, cache=cache)
+            hip(idx[:, :1], cache=cache)
+        assert seen.pop() is native
+
+
 def test_other_forms_take_the_general_step(monkeypatch):
     """A hook inside a block and autograd keep the module calls, with the same
     results; so does autocast, which their step kernel refuses."""
