@@ -22,7 +22,8 @@
 // Range: with x1 about 2^-9 x and x2 2^-18 x, values down to 2^-108 keep all
 // 24 bits (below, the parts run into the subnormals). Infinities, NaN and
 // values that round to a bf16 infinity make the element's sum NaN or
-// infinite here; the epilogue recomputes such elements with plain fp32 fmas.
+// infinite here; a wave that ends with such an element computes its part of
+// the tile again with fp32 MFMAs (plain_products).
 #pragma once
 
 #include "mhs_common.hpp"
@@ -166,6 +167,59 @@ struct GemmLoader {
   }
 };
 
+// 4 of the 8 k's from k of row r of one operand (rows rows, k's below k_end):
+// the lane's operands of 4 fp32 MFMAs, lanes 32-63 taking the second 4 k's.
+template <bool KMAJOR>
+__device__ __forceinline__ void load_plain(float (&v)[4], const float* p, long long ld, int r,
+                                           int rows, int k, int k_end) {
+  k += 4 * ((threadIdx.x >> 5) & 1);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) v[t] = 0.f;
+  if (r >= rows || k >= k_end) return;
+  if constexpr (KMAJOR) {   // K a multiple of 4: a whole float4
+    f4_to(v, *reinterpret_cast<const float4*>(p + (long long)r * ld + k));
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (k + t < k_end) v[t] = p[(long long)(k + t) * ld + r];
+  }
+}
+
+// The wave's FM x FN fragments from row m, column n, over k's k_first ..
+// k_end - 1, with fp32 MFMAs from global memory: a lane's operands are row (or
+// column) lane % 32, k lane / 32, and the sum's elements lie as the bf16
+// products' do. For the waves that meet infinities, NaN or parts that
+// overflow; bound by the fp32 matrix rate. 8192 x 1464 x 1432 of NaN: 490 to 560 us
+// with the bf16 products before it, against 21 to 32 ms by a serial fma loop
+// per element and 265 us by the library.
+template <bool AK, bool BK, int FM, int FN>
+__device__ __forceinline__ void plain_products(f32x16 (&acc)[FM][FN], const GemmArgs& g, int m,
+                                               int n, int k_first, int k_end) {
+  m += threadIdx.x & 31;
+  n += threadIdx.x & 31;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+#pragma unroll 1
+  for (int k = k_first; k < k_end; k += 8) {
+    float a[FM][4], b[FN][4];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) load_plain<AK>(a[i], g.A, g.lda, m + 32 * i, g.M, k, k_end);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) load_plain<BK>(b[j], g.B, g.ldb, n + 32 * j, g.N, k, k_end);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][t], b[j][t], acc[i][j], 0, 0, 0);
+  }
+}
+
 // One 128 x 128 tile per block, 2 x 2 waves of 64 x 64 (or 64 x 64 of 32 x 32,
 // for products of few tiles), k 16 deep and double
 // buffered: while a wave multiplies a tile it splits the next one into the
@@ -279,6 +333,17 @@ gemm3_kernel(GemmArgs g) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][j][e] = -acc[i][j][e];
 
+  float odd = 0.f;   // NaN once an element is not finite
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) odd = __builtin_fmaf(acc[i][j][e], 0.f, odd);
+  if (__builtin_amdgcn_ballot_w64(odd != odd) != 0)
+    plain_products<AK, BK>(acc, g, m0 + wm * (BM / 2), n0 + wn * (BN / 2), k_first,
+                           k_first + k_len);
+
   // A fragment's element e of lane l: row 8 (e / 4) + 4 (l / 32) + e % 4,
   // column l % 32.
   float* const cb = g.C + (long long)blockIdx.y * g.M * g.ldc;
@@ -288,24 +353,6 @@ gemm3_kernel(GemmArgs g) {
     for (int j = 0; j < FN; ++j) {
       const int n = n0 + wn * (BN / 2) + j * 32 + (lane & 31);
       const int mb = m0 + wm * (BM / 2) + i * 32 + 4 * (lane >> 5);
-      float odd = 0.f;   // NaN once an element is not finite
-#pragma unroll
-      for (int e = 0; e < 16; ++e) odd = __builtin_fmaf(acc[i][j][e], 0.f, odd);
-      if (odd != odd) {
-        // Infinities, NaN or overflowing parts: plain fp32 for those elements.
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = mb + 8 * (e / 4) + e % 4;
-          if (acc[i][j][e] * 0.f == 0.f || m >= g.M || n >= g.N) continue;
-          float s = 0.f;
-          for (int k = k_first; k < k_first + k_len; ++k) {
-            const float av = AK ? g.A[(long long)m * g.lda + k] : g.A[(long long)k * g.lda + m];
-            const float bv = BK ? g.B[(long long)n * g.ldb + k] : g.B[(long long)k * g.ldb + n];
-            s = __builtin_fmaf(av, bv, s);
-          }
-          acc[i][j][e] = s;
-        }
-      }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int m = mb + 8 * (e / 4) + e % 4;

@@ -95,6 +95,48 @@ def test_infinities_and_nan_come_out_as_in_fp32():
     assert torch.equal(torch.isinf(out), inf) and torch.equal(out[inf], ref[inf])
 
 
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("m,n,k", [(33, 36, 20), (129, 132, 100), (257, 128, 8192)])
+def test_non_finite_elements_of_every_form(form, m, n, k):
+    """Infinities, NaN and values whose parts overflow, in tiles with edges and
+    a split of k: the other elements keep their values."""
+    print(f"[case] non-finite gemm {form} {m}x{n}x{k}", flush=True)
+    f = FORMS[form]
+    a, b = _operands(f, m, n, k)
+    ka, kb = (a.t() if f == GEMM_TN else a), (b if f == GEMM_NT else b.t())   # rows by k
+    ka[m - 1, k - 1], ka[2, 0], kb[n - 2, k // 2] = float("nan"), float("inf"), -float("inf")
+    ka[5, 1], ka[6] = 3.4e38, 0.0
+    kb[:, 1] *= 1e-3
+    ref = _ref(a.double(), b.double(), f)
+    out = torch.empty(m, n, device=DEV)
+    _call(a, b, f, out)
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(torch.isinf(out), inf) and torch.equal(out.double()[inf], ref[inf])
+    fin = torch.isfinite(ref)
+    bound = (6 * k / 16 + 40) * 2.0 ** -23 * _ref(a.double().abs(), b.double().abs(), f)
+    assert ((out.double() - ref).abs() <= bound)[fin].all()
+
+
+def test_non_finite_products_stay_fast():
+    """All NaN: the recomputation is bound by the fp32 matrix rate, a few times
+    the finite product (and not the hundreds of a loop per element)."""
+    a, b = _operands(GEMM_NT, 2048, 1464, 1432)
+    out = torch.empty(2048, 1464, device=DEV)
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    times = []
+    for x in (a, torch.full_like(a, float("nan"))):
+        _call(x, b, GEMM_NT, out)
+        start.record()
+        for _ in range(3):
+            _call(x, b, GEMM_NT, out)
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end))
+    assert torch.isnan(out).all()
+    assert times[1] < 15 * times[0], times
+
+
 @pytest.mark.parametrize("scale", [1e-12, 1e-19, 1e15])
 def test_scales(scale):
     a, b = (v * scale for v in _operands(GEMM_NT, 130, 128, 256))
