@@ -19,11 +19,15 @@
 // kGemmFlip k tiles: the roundings of neighbouring runs cancel (mean error
 // 1e-8, rms 2.2e-5; an fp32 rocBLAS product 5e-9 and 2.6e-5).
 //
-// Range: with x1 about 2^-9 x and x2 2^-18 x, values down to 2^-108 keep all
-// 24 bits (below, the parts run into the subnormals). Infinities, NaN and
-// values that round to a bf16 infinity make the element's sum NaN or
-// infinite here; a wave that ends with such an element computes its part of
-// the tile again with fp32 MFMAs (plain_products).
+// Range: with x1 about 2^-9 x and x2 2^-18 x, values down to 2^-110 keep all
+// 24 bits (below, the parts run into the subnormals). A thread ORs the leading
+// parts that it stages; where all of them lie below 2^-95 and not all are
+// zero, the block computes its tile again with fp32 MFMAs (plain_products). A
+// smaller value among larger ones of its row loses what is below their last
+// bits; values below 2^-134, among themselves too, count as zeros. Infinities,
+// NaN and values that round to a bf16 infinity make the element's sum NaN or
+// infinite: a wave that ends with such an element computes its part of the
+// tile again likewise.
 #pragma once
 
 #include "mhs_common.hpp"
@@ -64,7 +68,8 @@ __host__ __device__ constexpr int gemm_lds_bytes(int BM, int BN) {
 }
 
 // 8 consecutive k of one row, split: the three parts as 16-byte operands.
-__device__ __forceinline__ void split8(const float (&v)[8], bf16x8 (&p)[3]) {
+// seen: the leading parts ORed in.
+__device__ __forceinline__ void split8(const float (&v)[8], bf16x8 (&p)[3], unsigned& seen) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     f32x2 r = {v[2 * i], v[2 * i + 1]};
@@ -73,13 +78,22 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8 (&p)[3]) {
       const bf16x2 h = __builtin_convertvector(r, bf16x2);
       p[q][2 * i] = h[0];
       p[q][2 * i + 1] = h[1];
+      const unsigned u = __builtin_bit_cast(unsigned, h);
+      if (q == 0) seen |= u;
       if (q < 2) {
-        const unsigned u = __builtin_bit_cast(unsigned, h);
         r[0] -= __uint_as_float(u << 16);
         r[1] -= __uint_as_float(u & 0xffff0000u);
       }
     }
   }
+}
+
+// Whether the two bf16's of `seen`, an OR of parts, have exponents below
+// 2^-95's and are not both zero (of exponent fields below 32 and others, the OR
+// tells which: no sum carries).
+__device__ __forceinline__ bool all_tiny(unsigned seen) {
+  seen = (seen | seen >> 16) & 0x7fffu;
+  return seen != 0 && seen < (32u << 7);
 }
 
 // The staging of one operand's R x 16 tile: one task per thread, a task being
@@ -102,6 +116,7 @@ struct GemmLoader {
   unsigned off[T];     // byte offset of the task at k tile 0, or kOOB
   int kpos[T];         // first k of the task within a tile
   int lds[T];          // byte offset in a plane
+  unsigned seen = 0;   // the leading parts staged so far, ORed
   __device__ __forceinline__ GemmLoader(const float* p, long long ld_, int r0, int rows,
                                         long long k_first)
       : ld(ld_), width(rows - r0) {
@@ -151,7 +166,7 @@ struct GemmLoader {
       }
     }
   }
-  __device__ __forceinline__ void store(char* tile, const float (&w)[T][8], unsigned sign) const {
+  __device__ __forceinline__ void store(char* tile, const float (&w)[T][8], unsigned sign) {
     if (!mine()) return;
 #pragma unroll
     for (int i = 0; i < T; ++i) {
@@ -159,7 +174,7 @@ struct GemmLoader {
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(__float_as_uint(w[i][e]) ^ sign);
       bf16x8 p[3];
-      split8(v, p);
+      split8(v, p, seen);
 #pragma unroll
       for (int q = 0; q < 3; ++q)
         *reinterpret_cast<bf16x8*>(tile + q * gemm_plane_bytes(R) + lds[i]) = p[q];
@@ -257,8 +272,8 @@ gemm3_kernel(GemmArgs g) {
   const int k_len = min(g.K - k_first, g.kt_per_split * kGemmBK);
   const int nk = (k_len + kGemmBK - 1) / kGemmBK;
 
-  const GemmLoader<BM, AK, false> la(g.A, g.lda, m0, g.M, k_first);
-  const GemmLoader<BN, BK, true> lb(g.B, g.ldb, n0, g.N, k_first);
+  GemmLoader<BM, AK, false> la(g.A, g.lda, m0, g.M, k_first);
+  GemmLoader<BN, BK, true> lb(g.B, g.ldb, n0, g.N, k_first);
   float va[la.T][8], vb[lb.T][8];
   f32x16 acc[FM][FN];
 #pragma unroll
@@ -340,7 +355,12 @@ gemm3_kernel(GemmArgs g) {
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) odd = __builtin_fmaf(acc[i][j][e], 0.f, odd);
-  if (__builtin_amdgcn_ballot_w64(odd != odd) != 0)
+  // (The loop ended on a barrier: LDS is free.)
+  if (lane == 0) lds_f[wave] = 0.f;
+  if (all_tiny(la.seen) || all_tiny(lb.seen)) lds_f[wave] = 1.f;
+  __syncthreads();
+  const float4 tiny = *reinterpret_cast<const float4*>(lds_f);
+  if (__builtin_amdgcn_ballot_w64(odd != odd || tiny.x + tiny.y + tiny.z + tiny.w != 0.f) != 0)
     plain_products<AK, BK>(acc, g, m0 + wm * (BM / 2), n0 + wn * (BN / 2), k_first,
                            k_first + k_len);
 

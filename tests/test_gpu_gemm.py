@@ -145,6 +145,32 @@ def test_scales(scale):
     _assert_bounded(out, a, b, GEMM_NT, 256)
 
 
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("m,n,k", [(33, 36, 20), (200, 132, 300), (257, 128, 8192)])
+@pytest.mark.parametrize("scale", [1e-30, 1e-34, 1e-37])
+def test_small_operands_keep_their_bits(form, m, n, k, scale):
+    """Rows of one operand whose bf16 parts would run into the subnormals (the
+    other operand large, so that the results do not): all rows, and one. The
+    bar is that of the plain fp32 products which such tiles take: a sum of k
+    terms in any order, sqrt(k) / 2 roundings of at most 2^-24, with a margin
+    of 2, relative to the 2-norm."""
+    f = FORMS[form]
+    for which in ("a", "b"):
+        for rows in (slice(None), slice(3, 4)):
+            a, b = _operands(f, m, n, k)
+            ka, kb = (a.t() if f == GEMM_TN else a), (b if f == GEMM_NT else b.t())
+            small, large = (ka, kb) if which == "a" else (kb, ka)
+            small[rows] *= scale
+            large *= 1e20
+            out = torch.empty(m, n, device=DEV)
+            _call(a, b, f, out)
+            got, ref = out.double(), _ref(a.double(), b.double(), f)
+            if which == "b":
+                got, ref = got.t(), ref.t()
+            rel = (got - ref)[rows].norm() / ref[rows].norm()
+            assert rel <= k ** 0.5 * 2.0 ** -24 + 2.0 ** -23, (which, rows, rel.item())
+
+
 def test_linear_gradients():
     """A layer large enough for the HIP products in every direction."""
     rows, k, n = 2048, 640, 1464
