@@ -470,8 +470,7 @@ int mhs_rmsnorm_bwd_f32(const float* dy, const float* x, const float* weight, co
  * aligned pointer. Infinities and NaN come out as in plain fp32. Deterministic.
  *
  * mhs_gemm_workspace_bytes: the device workspace (256-byte aligned) of a
- * product, 0 for none, -1 for invalid sizes. With a workspace, c must be
- * 16-byte aligned and ldc a multiple of 4. mhs_gemm_preferred: 1 where the
+ * product, 0 for none, -1 for invalid sizes. mhs_gemm_preferred: 1 where the
  * product is faster than a BLAS library's fp32 one (large products), else 0.
  */
 #define MHS_GEMM_NT 0

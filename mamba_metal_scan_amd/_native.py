@@ -1164,8 +1164,6 @@ def _gemm_into(a: torch.Tensor, b: torch.Tensor, form: int, out: torch.Tensor,
     if not lib.mhs_gemm_preferred(m, n, k):
         return False
     nbytes = int(lib.mhs_gemm_workspace_bytes(m, n, k))
-    if nbytes and (out.stride(0) % 4 or out.data_ptr() % 16):
-        return False
     with _on(a.device):
         ws = torch.empty(nbytes, dtype=torch.uint8, device=a.device) if nbytes else None
         rc = lib.mhs_gemm_f32(form, _ptr(a), a.stride(0), _ptr(b), b.stride(0), _ptr(out),

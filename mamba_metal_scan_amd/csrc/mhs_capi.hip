@@ -1632,14 +1632,13 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
   const int cus = device_cus();
   const int kt = (int)((K + mhs::kGemmBK - 1) / mhs::kGemmBK);
   const int least = (int)((K + kGemmMaxChain - 1) / kGemmMaxChain);
-  // The reduction reads whole float4s: other widths are not split.
-  const int most = N % 4 == 0 ? std::max(least, std::min(kGemmMaxSplits, kt / 8)) : 1;
+  const int most = std::max(least, std::min(kGemmMaxSplits, kt / 8));
   double best = 0;
   for (const int tile : {mhs::kGemmTile, mhs::kGemmSmallTile}) {
     const int64_t gm = (M + tile - 1) / tile, gn = (N + tile - 1) / tile;
     if (gm * gn > 0x7FFFFFFF) continue;
     const double per_kt = tile == mhs::kGemmTile ? 0.6 : 0.25, alone = std::max(per_kt, 0.45);
-    for (int s = std::min(least, most); s <= most; ++s) {
+    for (int s = least; s <= most; ++s) {
       const double rounds = std::ceil((double)gm * gn * s / cus);
       const double us = std::max(rounds * per_kt, alone) * (kt / (double)s + 4) +
                         (s > 1 ? (2 * s + 1) * (double)M * N * 4 / 4.8e6 + 4 : 0);
@@ -1721,8 +1720,6 @@ int mhs_gemm_f32(int form, const float* a, int64_t lda, const float* b, int64_t 
   g.grid_m = p.grid_m;
   g.grid_n = p.grid_n;
   if (p.splits > 1) {
-    if (ldc % 4 || !aligned16(c))
-      return fail(MHS_EINVAL, "a split product needs c 16-byte aligned and ldc a multiple of 4");
     const size_t need = (size_t)p.splits * m * n * 4;
     if (!workspace || workspace_bytes < need)
       return fail(MHS_EINVAL, "workspace too small: %zu < %zu bytes", workspace_bytes, need);
@@ -1743,10 +1740,18 @@ int mhs_gemm_f32(int form, const float* a, int64_t lda, const float* b, int64_t 
                      dim3(mhs::kGemmThreads), mhs::gemm_lds_bytes(p.tile, p.tile), s, g);
   rc = check_launch("matrix product kernel");
   if (rc || p.splits == 1) return rc;
-  const long long n4 = (long long)m * (n / 4);
-  hipLaunchKernelGGL(mhs::gemm_reduce_kernel<>, dim3((unsigned)std::min<long long>((n4 + 255) / 256, 4096)),
-                     dim3(256), 0, s, g.C, c, p.splits, (long long)m, (int)(n / 4),
-                     (long long)(ldc / 4), accumulate);
+  // Whole float4s where c's rows hold and start at such.
+  const bool vec = n % 4 == 0 && ldc % 4 == 0 && aligned16(c);
+  const long long count = (long long)m * (vec ? n / 4 : n);
+  const dim3 grid((unsigned)std::min<long long>((count + 255) / 256, 4096));
+  if (vec)
+    hipLaunchKernelGGL(mhs::gemm_reduce_kernel<float4>, grid, dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(g.C), reinterpret_cast<float4*>(c),
+                       p.splits, (long long)m, (int)(n / 4), (long long)(ldc / 4), accumulate);
+  else
+    hipLaunchKernelGGL(mhs::gemm_reduce_kernel<float>, grid, dim3(256), 0, s,
+                       static_cast<const float*>(g.C), c, p.splits, (long long)m, (int)n,
+                       (long long)ldc, accumulate);
   return check_launch("matrix product reduction kernel");
 }
 

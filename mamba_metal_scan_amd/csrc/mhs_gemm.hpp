@@ -397,28 +397,26 @@ concat3_kernel(const float4* __restrict__ a, const float4* __restrict__ b,
   else if (i < na + nb + nc) out[i] = c[i - na - nb];
 }
 
+__device__ __forceinline__ float add(float a, float b) { return a + b; }
+__device__ __forceinline__ float4 add(float4 a, float4 b) {
+  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
 // out (M, N; rows ldc apart) = the sum of the split-K partials (splits, M,
-// N), in split order (+ out). N a multiple of 4, rows 16-byte aligned.
-template <int UNUSED = 0>
+// N), in split order (+ out). V: float4 (N and ldc in float4s; rows 16-byte
+// aligned), or float for any width.
+template <class V>
 __global__ void __launch_bounds__(256)
-gemm_reduce_kernel(const float* __restrict__ part, float* __restrict__ out, int splits, long long M,
-                   int N4, long long ldc4, int accumulate) {
-  const long long n = M * N4;
-  const float4* p = reinterpret_cast<const float4*>(part);
-  float4* o = reinterpret_cast<float4*>(out);
+gemm_reduce_kernel(const V* __restrict__ part, V* __restrict__ out, int splits, long long M,
+                   int N, long long ldc, int accumulate) {
+  const long long n = M * N;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n;
        i += (long long)gridDim.x * 256) {
-    const long long at = ldc4 == N4 ? i : i / N4 * ldc4 + i % N4;
-    float4 s = p[i];
-    for (int k = 1; k < splits; ++k) {
-      const float4 t = p[k * n + i];
-      s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-    }
-    if (accumulate) {
-      const float4 t = o[at];
-      s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-    }
-    o[at] = s;
+    const long long at = ldc == N ? i : i / N * ldc + i % N;
+    V s = part[i];
+    for (int k = 1; k < splits; ++k) s = add(s, part[k * n + i]);
+    if (accumulate) s = add(s, out[at]);
+    out[at] = s;
   }
 }
 

@@ -83,6 +83,27 @@ def test_widths_that_are_no_multiple_of_four(form, m, n, k):
     _assert_bounded(out, a, b, f, k)
 
 
+@pytest.mark.parametrize("form,m,n,k", [("nt", 33, 7, 8192), ("nn", 129, 131, 9000),
+                                        ("tn", 130, 642, 9001), ("tn", 64, 64, 20000)])
+def test_long_sums_of_any_width_are_split(form, m, n, k):
+    """More than 4096 k's are summed in several chains at any width and row
+    stride of c: the error stays below a plain fp32 product's (one chain of
+    MFMA additions of 32768 has 1.5 times it)."""
+    print(f"[case] gemm {form} {m}x{n}x{k}", flush=True)
+    f = FORMS[form]
+    a, b = _operands(f, m, n, k)
+    ref = _ref(a.double(), b.double(), f)
+    lib = (_native._mm(a, b, f).double() - ref).norm() / ref.norm()
+    for pad in (0, 1):
+        out = torch.full((m, n + pad), float("nan"), device=DEV)[:, :n]
+        assert _call(a, b, f, out) >= 2 * m * n * 4
+        _assert_bounded(out, a, b, f, k)
+        rel = (out.double() - ref).norm() / ref.norm()
+        assert rel <= 1.1 * lib, (rel.item(), lib.item())
+        _call(a, b, f, out.fill_(0.5), accumulate=True)
+        _assert_bounded(out, a, b, f, k, extra=0.5)
+
+
 def test_infinities_and_nan_come_out_as_in_fp32():
     a, b = _operands(GEMM_NT, 200, 140, 64)
     a[3, 5], a[7, 9], b[11, 2], a[20, 1] = float("inf"), float("nan"), -float("inf"), 3.4e38

@@ -386,3 +386,12 @@ def test_rmsnorm_argument_errors():
     assert rc == MHS_EINVAL and "aligned" in _err(lib)
     rc = lib.mhs_rmsnorm_bwd_f32(a, a, a, None, None, b, a, b, ws, 8192, 640, None)
     assert rc == MHS_EINVAL and "null" in _err(lib)
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 64, 4097), (642, 1284, 32768), (641, 1283, 32768),
+                                   (7, 3, 9001)])
+def test_product_splits_bound_the_chains(m, n, k):
+    """The workspace holds one partial per split: no chain of more than 4096
+    k's at any width."""
+    splits = _native.library().mhs_gemm_workspace_bytes(m, n, k) // (m * n * 4)
+    assert splits >= -(-k // 4096)
