@@ -1622,6 +1622,7 @@ namespace {
 // 1.62e-6; at 32768 in one chain 3.0e-6 against 2.0e-6).
 constexpr int kGemmMaxChain = 4096;
 constexpr int kGemmMaxSplits = 32;
+constexpr int kGemmGridSplits = 32768;   // and longer chains past 2^27 k's: blockIdx.y's range
 
 struct GemmPlan {
   int tile = 0, grid_m = 0, grid_n = 0, splits = 1, kt_per_split = 0;
@@ -1631,7 +1632,7 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
   GemmPlan p;
   const int cus = device_cus();
   const int kt = (int)((K + mhs::kGemmBK - 1) / mhs::kGemmBK);
-  const int least = (int)((K + kGemmMaxChain - 1) / kGemmMaxChain);
+  const int least = (int)std::min<int64_t>((K + kGemmMaxChain - 1) / kGemmMaxChain, kGemmGridSplits);
   const int most = std::max(least, std::min(kGemmMaxSplits, kt / 8));
   double best = 0;
   for (const int tile : {mhs::kGemmTile, mhs::kGemmSmallTile}) {

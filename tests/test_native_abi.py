@@ -389,9 +389,9 @@ def test_rmsnorm_argument_errors():
 
 
 @pytest.mark.parametrize("m,n,k", [(64, 64, 4097), (642, 1284, 32768), (641, 1283, 32768),
-                                   (7, 3, 9001)])
+                                   (7, 3, 9001), (4, 4, 1 << 27), (4, 4, 1 << 30)])
 def test_product_splits_bound_the_chains(m, n, k):
     """The workspace holds one partial per split: no chain of more than 4096
-    k's at any width."""
+    k's at any width (up to 2^27 of them), and no more splits than a grid's y."""
     splits = _native.library().mhs_gemm_workspace_bytes(m, n, k) // (m * n * 4)
-    assert splits >= -(-k // 4096)
+    assert min(-(-k // 4096), 32768) <= splits <= 65535
