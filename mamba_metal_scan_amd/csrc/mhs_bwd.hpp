@@ -149,6 +149,16 @@ __host__ __device__ constexpr bool bwd_row_partial(int NPL, bool CARRY, int SWEE
   return bwd_relabel(NPL, CARRY) && SWEEP == 0;
 }
 
+// Whether dAneg is summed chunk by chunk before it joins the walk's sum. One
+// chain of additions per segment grows its rounding error with the segment's
+// length; the segments of these plans may be up to six times as long as those
+// of segments_for (relative 2-norm error at 4x1024x1024x64: 3.3e-7 in six
+// segments, in two 4.6e-7 in one chain and 2.6e-7 so; no register more, 320
+// us a forward and backward either way). The other plans keep their segments
+// that short (2x1024x1920x16: 132 -> 135 us, 144 before least_segments; the
+// sums would cost the dense grids 0.2 to 0.6%).
+__host__ __device__ constexpr bool bwd_chunk_sums(int NPL, int G) { return NPL == 4 || G > 4; }
+
 // The layout of the backward's channel-major tiles (dt, dy, x, dt*x): padded
 // in the gradient kernels, whose walk switches staging buffers every chunk
 // (one address add per tile row and switch, not per quad); swizzled in the
@@ -288,6 +298,17 @@ bwd_kernel(BwdArgs a) {
   // carries u, so that G_t = dy_t C_t + u and dA_t h_{t-1} G_t = u_t h_{t-1}
   // each take one operation.
   float an[NPL], a2[NPL], u[NPL], acc[NPL];
+  // acc += dt * qv of step k; CS: by way of the chunk's own sum.
+  constexpr bool CS = bwd_chunk_sums(NPL, G);
+  float part[NPL];
+  const auto add_daneg = [&](int j, int k, float dtv, float qv) {
+    if constexpr (!CS) {
+      acc[j] = __builtin_fmaf(dtv, qv, acc[j]);
+    } else {
+      part[j] = k == kSteps - 1 ? dtv * qv : __builtin_fmaf(dtv, qv, part[j]);
+      if (k == 0) acc[j] += part[j];
+    }
+  };
 #pragma unroll
   for (int j = 0; j < NPL; ++j) {
     const int nj = j ^ sw;
@@ -705,7 +726,7 @@ bwd_kernel(BwdArgs a) {
               s1 = __builtin_fmaf(gk[j], Bq[s][j], s1);
             }
             s2 = __builtin_fmaf(an[j], qv, s2);
-            acc[j] = __builtin_fmaf(dts[s], qv, acc[j]);
+            add_daneg(j, kk, dts[s], qv);
           }
           s1q[s] = s1;
           s2q[s] = s2;
@@ -869,7 +890,7 @@ bwd_kernel(BwdArgs a) {
               s1 = __builtin_fmaf(gk[j], Bq[s][j], s1);
             }
             s2 = __builtin_fmaf(an[j], qv, s2);
-            acc[j] = __builtin_fmaf(dts[s], qv, acc[j]);
+            add_daneg(j, k, dts[s], qv);
           }
           s1q[s] = s1;
           s2q[s] = s2;

@@ -226,8 +226,9 @@ struct PassRate {
 //   10x700x740x32     94 -> 74 / 204 -> 150    3x2000x343x4   36 -> 26 / 61 -> 35
 constexpr int kMaxAutoSegments = 64, kMaxAutoUnits = 128;
 
+// most: chunks per segment at most (0: any).
 Segments least_segments(int64_t blocks, int nch, int cus, int npl, int G, bool fwd,
-                        double unit_bytes) {
+                        double unit_bytes, int most) {
   // us per chunk, fitted to the times of 19 grids at 12 d_states split 1 to 8
   // ways. Up to four waves a block has a wave per SIMD, beyond that two.
   const bool two = npl <= 2, thin = two && G <= 4;
@@ -260,6 +261,7 @@ Segments least_segments(int64_t blocks, int nch, int cus, int npl, int G, bool f
       r.nseg = (nch + r.cps - 1) / r.cps;
       r.nunits = (nch + r.ups - 1) / r.ups;
       const double carried = (double)(r.nseg - 1) * cu;
+      if (most > 0 && r.cps > most) continue;
       if (carried > kMaxAutoUnits || carried * unit_bytes + 512 > MHS_NOALLOC_SCRATCH_BYTES)
         continue;
       double us = main.us((double)blocks * r.nseg, r.cps, cus);
@@ -313,7 +315,10 @@ bool sparse_segments(int64_t batch, int64_t D, int64_t N, int nch, bool fwd, Seg
       out = e.s;
       return true;
     }
-  out = least_segments(blocks, nch, cus, npl, G, fwd, (double)batch * D * (N + 1) * 4);
+  // dAneg's chain of additions no longer than segments_for's (bwd_chunk_sums).
+  const int most = fwd || mhs::bwd_chunk_sums(npl, G)
+                       ? 0 : segments_for(batch, D, nch, kBwdBlocksPerCU).cps;
+  out = least_segments(blocks, nch, cus, npl, G, fwd, (double)batch * D * (N + 1) * 4, most);
   memo[next] = Entry{batch, D, (int)N, nch, cus, npl, fwd, out};
   next = (next + 1) % 8;
   return true;

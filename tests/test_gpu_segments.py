@@ -9,12 +9,14 @@ start state is folded from its predecessors' instead of walked), bf16 outputs
 """
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
 
 from helpers import rel_err
 from mamba_metal_scan_amd import _native, selective_scan_gated, selective_scan_hip
+from oracle import oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -132,3 +134,24 @@ def test_dense_gradients_of_middle_states_equal_two_states_per_lane(n, chunk, ga
     finally:
         _native.set_variant(0)
     _compare(auto, two, False)
+
+
+@pytest.mark.parametrize("bt,t,d,n,eighth", [(4, 512, 1536, 32, 8), (2, 2048, 1792, 16, 19),
+                                            (4, 1024, 1024, 64, 11)])
+def test_long_segments_do_not_add_error(bt, t, d, n, eighth):
+    """dAneg's error against float64 where the automatic split takes fewer
+    segments than those of `eighth` chunks each that the grid's
+    blocks per CU would give. Bar (relative 2-norm): a chain of m = 16 eighth
+    additions of terms of any sign rounds each by about 0.4 2^-24 of a running
+    sum that grows as the root of its length, 0.4 2^-24 sqrt(m / 2) in all,
+    and 2 2^-24 for the terms: 3.1e-7, 4.1e-7, 3.4e-7. (One chain over the
+    longer segments: 4.6e-7, 4.5e-7, 4.7e-7.)"""
+    print(f"[case] dAneg error {bt}x{t}x{d}x{n}", flush=True)
+    arrs = oracle.make_inputs(bt, t, d, n, seed=1, style="bench")
+    dy = np.random.default_rng(2).standard_normal((bt, t, d), dtype=np.float32)
+    leaves = [torch.from_numpy(a).to(DEV).requires_grad_() for a in arrs]
+    y = selective_scan_hip(*leaves, chunk=16)
+    da = torch.autograd.grad(y, leaves[2], torch.from_numpy(dy).to(DEV))[0]
+    ref = oracle.scan_bwd(*arrs, dy)[2]
+    rel = np.linalg.norm(da.cpu().double().numpy() - ref) / np.linalg.norm(ref)
+    assert rel <= 2.0 ** -24 * (0.4 * (16 * eighth / 2) ** 0.5 + 2), rel
