@@ -136,7 +136,8 @@ xent_fwd_kernel(const float* __restrict__ logits, const long long* __restrict__ 
 
 // loss[0] = the sum of loss_rows over the count of targets that are not
 // ignore_index (0 / 0 = NaN, as the framework's mean); n_valid[0] = the count.
-// One block, in a fixed order: a launch where the framework takes four.
+// One block, in a fixed order: a launch where the framework takes four (8192
+// rows 6.7 against 18.7 us; past 131072 rows the four are the faster).
 constexpr int kXentMeanThreads = 1024;
 template <int UNUSED = 0>
 __global__ void __launch_bounds__(kXentMeanThreads)

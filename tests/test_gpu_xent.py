@@ -194,3 +194,30 @@ def test_mean_over_rows(rows):
     valid = (targets != -100).sum()
     assert n.item() == valid.item()
     assert abs(loss.item() - loss_rows.double().sum().item() / valid.item()) <= 1e-6
+
+
+@pytest.mark.parametrize("rows", [1 << 17, (1 << 17) + 1, 1 << 20])
+def test_mean_over_many_rows(rows):
+    """On both sides of the one-block mean's last row count, and far past it,
+    where one block would take nine times as long as the framework's sums."""
+    g = torch.Generator().manual_seed(rows)
+    loss_rows = torch.rand(rows, generator=g)
+    targets = torch.randint(0, 9, (rows,), generator=g)
+    targets[1::7] = -100
+    loss_rows[1::7] = 0.0
+    want = loss_rows.double().sum().item() / (targets != -100).sum().item()
+    lr, t = loss_rows.to(DEV), targets.to(DEV)
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    times = []
+    for f in (lambda: torch.ops.mamba_hip.xent_mean(lr, t, -100),
+              lambda: (lr.sum() / (t != -100).sum(), (t != -100).sum())):
+        loss, n = f()
+        assert n.dtype == torch.int64 and n.item() == (targets != -100).sum().item()
+        assert abs(loss.item() - want) <= 1e-6
+        start.record()
+        for _ in range(10):
+            f()
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end))
+    assert times[0] <= 4 * times[1], times
