@@ -104,8 +104,8 @@ def block_forward(x: torch.Tensor, delta: Optional[torch.Tensor], params: tuple,
     x_out = torch.empty_like(x) if delta is not None else x
     xz = x.new_empty((bt, t_len, 2 * d))
     h_last = x.new_empty((bt, d, n)) if want_state else None
-    saved = torch.empty(lib.mhs_block_saved_bytes(*sizes, consts[3], with_ckpt),
-                        dtype=torch.uint8, device=dev)
+    # (fp32, as its contents: saved-tensor hooks may convert what they pack)
+    saved = x.new_empty(lib.mhs_block_saved_bytes(*sizes, consts[3], with_ckpt) // 4)
     nbytes = lib.mhs_block_fwd_workspace_bytes(*sizes)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     with _native._on(dev):
@@ -115,6 +115,16 @@ def block_forward(x: torch.Tensor, delta: Optional[torch.Tensor], params: tuple,
             consts[3], with_ckpt, ws.data_ptr(), nbytes, _native._stream(dev))
     _native._check(rc, "mhs_block_fwd_f32")
     return x_out, out, xz, saved, h_last
+
+
+def _restored(t: torch.Tensor, align: int) -> torch.Tensor:
+    """A saved tensor as the kernels read it, whatever layout a saved-tensor
+    hook gave it back in."""
+    if t.dtype is not _f32:
+        raise TypeError(f"the block's saved tensors are float32; a saved-tensor hook returned "
+                        f"{t.dtype}")
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % align else t
 
 
 class BlockHIP(torch.autograd.Function):
@@ -133,6 +143,8 @@ class BlockHIP(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_x, g_out):
         x, xz, saved, *params = ctx.saved_tensors
+        saved = _restored(saved, 256)
+        x, xz, *params = (_restored(t, 16) for t in (x, xz, *params))
         need = ctx.needs_input_grad
         if g_out is None:
             g_out = torch.zeros_like(x)

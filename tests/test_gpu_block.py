@@ -7,6 +7,8 @@ Bar: 1e-4 max relative per tensor, the build's parity bar.
 """
 from __future__ import annotations
 
+import contextlib
+
 import pytest
 import torch
 
@@ -109,6 +111,45 @@ def test_frozen_weights_and_unused_outputs():
     x_out, _ = hip._native(xi, delta)
     x_out.sum().backward()
     assert torch.equal(xi.grad, torch.ones_like(x)) and torch.equal(delta.grad, xi.grad)
+
+
+@pytest.mark.parametrize("form", ["cpu", "strided", "offset", "bf16"])
+def test_saved_tensor_hooks(form):
+    """Hooks that move what the forward saved, give it back in another layout
+    or at another alignment, or keep it in bf16 (whatever is saved, floating
+    point or not, must survive as numbers)."""
+    print(f"[case] saved-tensor hooks {form}", flush=True)
+    hip, _ = _blocks(64, 96)
+    x = torch.randn(2, 33, 64, generator=torch.Generator().manual_seed(0)).to(DEV)
+    packed = []
+
+    def pack(t):
+        packed.append(t.dtype)
+        return t.to(torch.bfloat16) if form == "bf16" else t.cpu()
+
+    def unpack(t):
+        t = t.float().to(DEV)
+        if form == "strided":
+            return torch.stack([t, t], -1)[..., 0]
+        if form == "offset":
+            return torch.cat([t.new_zeros(5), t.flatten()])[5:].view(t.shape)
+        return t
+
+    def run(ctx):
+        xi = x.clone().requires_grad_()
+        hip.zero_grad(set_to_none=True)
+        with ctx:
+            out = hip(xi)
+        out.square().sum().backward()
+        return [out.detach(), xi.grad, *[p.grad for p in hip.parameters()]]
+    want = run(contextlib.nullcontext())
+    got = run(torch.autograd.graph.saved_tensors_hooks(pack, unpack))
+    assert packed and set(packed) == {torch.float32}
+    for i, (a, b) in enumerate(zip(got, want)):
+        if form == "bf16":
+            assert_close(f"output {i}", a, b, tol=0.1)
+        else:
+            assert torch.equal(a, b), i
 
 
 def test_hooks_subclasses_and_offset_views_take_the_module_path(monkeypatch):
