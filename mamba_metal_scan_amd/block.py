@@ -133,8 +133,10 @@ class BlockHIP(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, delta, consts, *params):
-        x_out, out, xz, saved, _ = block_forward(x, delta, params, consts, True, False)
-        ctx.save_for_backward(x_out, xz, saved, *params)
+        need = any(ctx.needs_input_grad)   # (a frozen block keeps nothing)
+        x_out, out, xz, saved, _ = block_forward(x, delta, params, consts, need, False)
+        if need:
+            ctx.save_for_backward(x_out, xz, saved, *params)
         ctx.consts = consts
         ctx.has_delta = delta is not None
         ctx.set_materialize_grads(False)

@@ -113,6 +113,22 @@ def test_frozen_weights_and_unused_outputs():
     assert torch.equal(xi.grad, torch.ones_like(x)) and torch.equal(delta.grad, xi.grad)
 
 
+def test_frozen_blocks_keep_no_checkpoints(monkeypatch):
+    """With autograd on and nothing to differentiate, as with it off: no
+    checkpoints are written, nothing is saved."""
+    hip, ref = _blocks(64, 96)
+    hip.requires_grad_(False)
+    seen = _calls(monkeypatch)
+    x = torch.randn(2, 33, 64, generator=torch.Generator().manual_seed(0))
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(packed.append, lambda t: t):
+        out = hip(x.to(DEV))
+    assert seen == [False] and packed == [] and not out.requires_grad
+    assert_close("out", out, ref(x.double()))
+    hip(x.to(DEV).requires_grad_())
+    assert seen == [False, True]
+
+
 @pytest.mark.parametrize("form", ["cpu", "strided", "offset", "bf16"])
 def test_saved_tensor_hooks(form):
     """Hooks that move what the forward saved, give it back in another layout
