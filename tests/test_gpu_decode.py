@@ -76,6 +76,38 @@ def test_token_matches_float64(monkeypatch, batch, over):
     assert seen == [True] * 3
 
 
+@pytest.mark.parametrize("batch,shift", [(4, 0.0), (8, -8.0)])
+def test_error_is_no_larger_than_the_modules(monkeypatch, batch, shift):
+    """A token of a 640-wide block from a given cache: the relative 2-norm
+    error of its logits, state and window against float64 beside that of the
+    module calls, which use the framework's softplus, sigmoid and exp and the
+    library's products. Bar: 1.2 times it (measured 0.5 to 1.0 of it)."""
+    print(f"[case] decode error batch {batch}", flush=True)
+    hip, ref = _models(d_model=640, d_inner=1432, n_layers=1)
+    with torch.no_grad():
+        for m in (hip, ref):
+            m.blocks[0].A.add_(shift)
+    ref = ref.to(DEV)
+    g = torch.Generator().manual_seed(batch)
+    start = {"h": torch.randn(batch, 1432, 16, generator=g).to(DEV),
+             "conv": torch.randn(batch, 1432, 3, generator=g).to(DEV)}
+    tok = torch.randint(0, 203, (batch, 1), generator=g).to(DEV)
+
+    def run(model, dtype):
+        cache = {"blocks": [{k: v.to(dtype, copy=True) for k, v in start.items()}]}
+        with torch.no_grad():
+            logits = model(tok, cache=cache)[0]
+        return [v.double() for v in (logits, cache["blocks"][0]["h"], cache["blocks"][0]["conv"])]
+    want = run(ref, torch.float64)
+    seen = _native_calls(monkeypatch)
+    native = run(hip, torch.float32)
+    assert seen == [True]
+    monkeypatch.setattr("mamba_metal_scan_amd.model.decode_step", lambda *a: None)
+    for name, a, b, w in zip(("logits", "h", "conv"), native, run(hip, torch.float32), want):
+        ea, eb = ((v - w).norm() / w.norm() for v in (a, b))
+        assert ea <= 1.2 * eb, (name, ea.item(), eb.item())
+
+
 def test_batches_on_both_sides_of_the_limit(monkeypatch):
     """The largest batch of the native token and the next, which takes the
     module calls; both follow the float64 step."""
