@@ -13,9 +13,12 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 
 from . import _native
+from .fused import mamba_inner
 from .linear import PLAIN
+from .norm import rms_norm_residual
 
 _WEIGHTS = struct.Struct("11Q4f")      # mhs_block_weights
 _GRADS = struct.Struct("10Q")          # mhs_block_grads
@@ -127,6 +130,29 @@ def _restored(t: torch.Tensor, align: int) -> torch.Tensor:
     return t.clone() if t.data_ptr() % align else t
 
 
+def _module_gradients(ctx, x: torch.Tensor, params: list, g_x, g_out) -> tuple:
+    """The backward's gradients by way of the functions of the module path run
+    again, for a caller that differentiates them: a graph over the products,
+    as that path's own backward leaves it (the kernels' Functions are first
+    order). Differentiated by aliases: x is an output of this node itself where
+    a delta was added, and the way to the weights must not lead through it."""
+    leaves = [t.view_as(t) for t in (x, *params)]
+    x, *params = leaves
+    norm_w, in_w, conv_w, conv_b, dt_w, dt_b, a, b_w, c_w, d_skip, out_w = params
+    eps, dt_min, dt_max, chunk = ctx.consts
+    res, h = rms_norm_residual(x, norm_w, eps)
+    out = F.linear(mamba_inner(F.linear(h, in_w), conv_w, conv_b, dt_w, dt_b, b_w, c_w, a, d_skip,
+                               dt_min, dt_max, chunk=chunk), out_w)
+    need = [i for i, t in enumerate(leaves) if t.requires_grad]
+    pairs = [(o, g) for o, g in ((res, g_x), (out, g_out)) if g is not None]
+    got = torch.autograd.grad([o for o, _ in pairs], [leaves[i] for i in need],
+                              [g for _, g in pairs], create_graph=True, allow_unused=True)
+    grads = [None] * len(leaves)
+    for i, g in zip(need, got):
+        grads[i] = g
+    return (grads[0], grads[0] if ctx.has_delta else None, None, *grads[1:])
+
+
 class BlockHIP(torch.autograd.Function):
     """(x + delta, out) of a block; delta None: (x, out). The gradients of both
     outputs reach x and delta in the norm's backward kernel."""
@@ -145,6 +171,8 @@ class BlockHIP(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_x, g_out):
         x, xz, saved, *params = ctx.saved_tensors
+        if torch.is_grad_enabled():   # create_graph
+            return _module_gradients(ctx, x, params, g_x, g_out)
         saved = _restored(saved, 256)
         x, xz, *params = (_restored(t, 16) for t in (x, xz, *params))
         need = ctx.needs_input_grad

@@ -140,6 +140,36 @@ def test_error_is_no_larger_than_the_modules():
         assert ea <= 1.3 * eb + 2.0 ** -23, (name, ea.item(), eb.item())
 
 
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_gradients_of_gradients_as_the_module_path_leaves_them(with_delta):
+    """create_graph: first-order gradients equal, and a penalty on the
+    projections' weight gradients has the gradients that the module path (a
+    hook on in_proj) gives it."""
+    print(f"[case] create_graph block delta {with_delta}", flush=True)
+    m = TinyMamba(MambaConfig(vocab_size=50, d_model=64, n_layers=2, d_ff=128,
+                              scan_impl="hip")).to(DEV)
+    block = m.blocks[1] if with_delta else m.blocks[0]
+    idx = torch.randint(0, 50, (2, 20), generator=torch.Generator().manual_seed(0)).to(DEV)
+    x = torch.randn(2, 20, 64, generator=torch.Generator().manual_seed(1)).to(DEV)
+    weights = (block.in_proj.weight, block.out_proj.weight)
+
+    def run():
+        loss = m(idx, idx)[1] if with_delta else block(x).square().mean()
+        first = torch.autograd.grad(loss, weights, create_graph=True)
+        penalty = sum(g.square().sum() for g in first)
+        second = torch.autograd.grad(penalty, weights, allow_unused=True)
+        return [*first, *[torch.zeros_like(w) if v is None else v
+                          for v, w in zip(second, weights)]]
+    native = run()
+    handles = [b.in_proj.register_forward_hook(lambda mod, i, o: None) for b in m.blocks]
+    modules = run()
+    for h in handles:
+        h.remove()
+    for i, (a, b) in enumerate(zip(native, modules)):
+        assert_close(f"gradient {i}", a, b, tol=2e-5)
+    assert native[2].abs().max() > 0
+
+
 def test_frozen_blocks_keep_no_checkpoints(monkeypatch):
     """With autograd on and nothing to differentiate, as with it off: no
     checkpoints are written, nothing is saved."""
