@@ -170,6 +170,7 @@ K_CH, K_STEPS, K_BC_PAD, K_SWEEP_MAX = 32, 16, 4, 2
 K_CM_ROW = 20                    # kCmRow: a row of the backward's padded channel-major tiles
 K_BC_GROUP2 = 4 * 16 + 16        # kBCGroup2: a state group of the row broadcast tile
 K_BC_GROUPQ = 4 * 16 + 8         # kBCGroupQ: a state group of the quad broadcast tile
+K_GEMM_PAD = 64                  # kGemmPad: between the halves of a product's LDS plane
 LDS_PER_CU = 160 * 1024          # gfx950
 VGPRS_PER_SIMD_LANE = 512        # wave64 VGPR file per SIMD lane (gfx950, no AGPR split used)
 
@@ -205,6 +206,13 @@ def scan_lds_bytes(kind: str, g: int, npl: int) -> int:
     return 4 * floats
 
 
+def gemm_lds_bytes(tile: int) -> int:
+    """Dynamic LDS per block of gemm3_kernel with tile x tile tiles: two
+    buffers of three bf16 planes per operand, each plane two halves of 16
+    bytes a row and K_GEMM_PAD."""
+    return 2 * 3 * 2 * 2 * (tile * 16 + K_GEMM_PAD)
+
+
 def resource_usage(verbose: bool = False) -> dict:
     """{demangled kernel name: {remark: value}} from a device-only compile of
     every source with the compiler's kernel-resource-usage remarks."""
@@ -235,8 +243,10 @@ def resource_usage(verbose: bool = False) -> dict:
     return {d.replace("mhs::", ""): rows[n] for n, d in zip(names, dem)}
 
 
-# The kernels of the benchmarked workloads (d_state 16: NPL 2, G 4; the
-# one-state-per-lane plan NPL 1, G 8 beside them), with what each one is.
+# The kernels of the benchmarked workloads (d_state 16: NPL 2, G 4; beside
+# them the one-state-per-lane plan NPL 1, G 8 and the four-state plans of
+# d_state 32 and 64), the products, the token's and the loss's, with what each
+# one is.
 AUDIT = [
     ("fwd_kernel<2, 4, 3, true, false, 0, 4>", "forward, checkpoint stride a multiple of 16",
      "fwd", 4, 2),
@@ -257,9 +267,34 @@ AUDIT = [
     ("fwd_kernel<1, 8, 4, true, false, 0, 4>", "forward, one state per lane", "fwd", 8, 1),
     ("bwd_kernel<1, 8, 4, false, false, 4, false, 0>", "backward, one state per lane",
      "bwd", 8, 1),
+    ("fwd_kernel<4, 8, 2, true, false, 0, 4>", "forward, d_state 64", "fwd", 8, 4),
+    ("bwd_kernel<4, 8, 2, false, false, 4, true, 0>", "backward, d_state 64, atomics", "bwd", 8,
+     4),
+    ("bwd_kernel<4, 4, 2, false, false, 4, false, 0>",
+     "backward, d_state 32, grids of a block per CU and more", "bwd", 4, 4),
     ("bwd_reduce_kernel<4>", "dB / dC / dAneg partial sums", None, 4, 0),
     ("zero_grads_kernel<0>", "zero fill before the atomics", None, 4, 0),
     ("step_kernel_vec<1, 4>", "decode step, d_state 16", None, 4, 0),
+    ("gemm3_kernel<true, true, 128>", "product NT, 128 x 128 tiles", "gemm", 4, 128),
+    ("gemm3_kernel<true, false, 128>", "product NN, 128 x 128 tiles", "gemm", 4, 128),
+    ("gemm3_kernel<false, false, 128>", "product TN, 128 x 128 tiles", "gemm", 4, 128),
+    ("gemm3_kernel<true, true, 64>", "product NT, 64 x 64 tiles", "gemm", 4, 64),
+    ("gemm3_kernel<true, false, 64>", "product NN, 64 x 64 tiles", "gemm", 4, 64),
+    ("gemm3_kernel<false, false, 64>", "product TN, 64 x 64 tiles", "gemm", 4, 64),
+    ("gemm_reduce_kernel<HIP_vector_type<float, 4u> >", "sum of a split product's partials",
+     None, 4, 0),
+    ("decode_product_kernel<0, 4, 2, 3>", "token, norm, in_proj and conv, batch 3 and 4", None,
+     4, 0),
+    ("decode_product_kernel<0, 8, 2, 2>", "the same, larger batches", None, 4, 0),
+    ("decode_product_kernel<1, 4, 1, 6>", "token, dt, B and C projections, batch 3 and 4", None,
+     4, 0),
+    ("decode_product_kernel<1, 8, 1, 2>", "the same, larger batches", None, 4, 0),
+    ("decode_product_kernel<2, 4, 1, 6>", "token, out_proj, batch 3 and 4", None, 4, 0),
+    ("decode_product_kernel<3, 4, 4, 3>", "token, norm and head, batch 3 and 4", None, 4, 0),
+    ("decode_product_kernel<3, 8, 4, 2>", "the same, larger batches", None, 4, 0),
+    ("decode_state_kernel<4>", "token, state update and gate", None, 4, 0),
+    ("xent_fwd_kernel<0>", "loss forward", None, 4, 0),
+    ("xent_bwd_kernel<true>", "loss backward", None, 4, 0),
 ]
 
 
@@ -274,7 +309,8 @@ def resource_table(usage: dict) -> list:
         if not hits:
             raise KeyError(f"no kernel {prefix} in the library's resource remarks")
         r = usage[hits[0]]
-        lds = scan_lds_bytes(kind, waves_per_block, npl) if kind else 0
+        lds = (gemm_lds_bytes(npl) if kind == "gemm"   # npl: the tile
+               else scan_lds_bytes(kind, waves_per_block, npl) if kind else 0)
         lds_waves = (f"{(LDS_PER_CU // lds) * waves_per_block // 4}" if lds else "-")
         out.append(f"| `{prefix}` | {what} | {r['VGPRs']} | {r['AGPRs']} | {r['TotalSGPRs']} | "
                    f"{r['ScratchSize [bytes/lane]']} | {r['VGPRs Spill']} / {r['SGPRs Spill']} | "
@@ -285,7 +321,7 @@ def resource_table(usage: dict) -> list:
 def write_resource_profile(path: Path) -> Path:
     """profiles/kernel_resources_gfx950.md: the register and LDS audit."""
     usage = resource_usage()
-    lines = ["# Scan kernels on gfx950: registers, scratch, LDS and the occupancy they allow",
+    lines = ["# Kernels on gfx950: registers, scratch, LDS and the occupancy they allow",
              "", "Made by", "",
              "    python3 -m mamba_metal_scan_amd.build --resource-usage "
              "profiles/kernel_resources_gfx950.md", "",
@@ -293,7 +329,7 @@ def write_resource_profile(path: Path) -> Path:
              "device-only build of the library's sources (the flags of `build.py`). "
              "`waves/SIMD (registers)` is the compiler's occupancy from VGPRs, SGPRs and the "
              "launch bounds; `LDS B/block` is the dynamic LDS the host launches each scan "
-             "kernel with (a forward that writes checkpoints; one that does not, as the "
+             "or product kernel with (a forward that writes checkpoints; one that does not, as the "
              f"prefill, leaves out the {scan_lds_bytes('fwd', 4, 2) - scan_lds_bytes('fwd_nock', 4, 2)} "
              "B of checkpoint tiles at d_state 16), and `waves/SIMD (LDS)` what "
              f"{LDS_PER_CU // 1024} KiB of LDS per CU "

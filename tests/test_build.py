@@ -53,6 +53,15 @@ def test_lds_sizes_of_the_training_plan():
     assert 3 * rp <= build.LDS_PER_CU and 3 * sweep <= 160 * 1024
 
 
+def test_product_lds_size():
+    """Two buffers of three planes per operand; three blocks of large tiles
+    fit a CU."""
+    pad = re.search(r"kGemmPad = (\d+);", (build.CSRC / "mhs_gemm.hpp").read_text())
+    assert int(pad.group(1)) == build.K_GEMM_PAD
+    assert build.gemm_lds_bytes(128) == 2 * 3 * 2 * 2 * (2048 + 64) == 50688
+    assert 3 * build.gemm_lds_bytes(128) <= build.LDS_PER_CU
+
+
 def test_dpp_hazard_check_finds_short_wait_states():
     """The build's check of the device assembly (build.dpp_hazards): a DPP
     read, in an inline-asm block, of a VGPR needs 2 wait states after a VALU
