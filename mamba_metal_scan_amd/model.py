@@ -371,20 +371,22 @@ class MambaBlock(nn.Module):
         return self.out_proj(y * F.silu(z))
 
 
-_METHODS = tuple(k for k, v in vars(MambaBlock).items() if callable(v) and k != "__init__")
+_METHODS = frozenset(k for k, v in vars(MambaBlock).items() if callable(v))
 
 
 def _own_methods(b: nn.Module) -> bool:
     """Whether b is a MambaBlock itself (not a wrapper or a subclass) that runs
     the class's methods, none of them set on the instance."""
-    return type(b) is MambaBlock and not any(k in b.__dict__ for k in _METHODS)
+    if torch.compiler.is_compiling():   # (does not trace the sets' operator)
+        return type(b) is MambaBlock and not any(k in b.__dict__ for k in _METHODS)
+    return type(b) is MambaBlock and not b.__dict__.keys() & _METHODS
 
 
 def _plain_block(b: nn.Module) -> bool:
     """Whether calling b.mix() in place of b(x) skips nothing: b runs the
     class's own methods, and neither b, its norm nor the module-global
     registries hold forward or backward hooks."""
-    return _own_methods(b) and no_hooks(b) and no_hooks(b.norm)
+    return _own_methods(b) and no_hooks(b) and no_hooks(b._modules["norm"])
 
 
 class TinyMamba(nn.Module):
@@ -446,7 +448,7 @@ class TinyMamba(nn.Module):
         """The logits of one embedded token per sequence against the cache as
         one native call, or None where that does not apply (see decode_step)."""
         if (torch.is_grad_enabled() or self.cfg.scan_impl == "torch" or not _hip_device(x)
-                or not all(_plain_block(b) for b in self.blocks)):
+                or not all(_own_methods(b) and no_hooks(b) for b in self.blocks)):
             return None
         return decode_step(self, x, cache)
 
