@@ -912,7 +912,8 @@ def bench_train(steps: int = 10, warmup: int = 3, size: str = "60M",
     import torch
     from mamba_metal_scan_amd import MambaConfig, TinyMamba
     from mamba_metal_scan_amd.gemm_tuning import TABLE, use_tuned_gemms
-    tuned = use_tuned_gemms()
+    # Every product of the HIP path's step is the package's own.
+    tuned = scan_impl == "torch" and use_tuned_gemms()
     torch.manual_seed(1337)
     dev = torch.device("cuda", 0)
     sz = TRAIN_SIZES[size]
@@ -951,7 +952,8 @@ def bench_train(steps: int = 10, warmup: int = 3, size: str = "60M",
            "config": f"TinyMamba {size} class ({model.count_params() / 1e6:.1f}M parameters: "
                      f"vocab 32768, d_model {sz['d_model']}, {sz['n_layers']} layers, d_state "
                      f"16), batch {bt} x seq {seq}, fp32, AdamW (fused), scan_impl={scan_impl}",
-           "gemm_solutions": TABLE.name if tuned else "library default"}
+           "gemm_solutions": ("HIP, three bf16 parts" if scan_impl != "torch"
+                              else TABLE.name if tuned else "library default")}
     del model, opt
     torch.cuda.empty_cache()
     return out

@@ -1768,7 +1768,14 @@ int mhs_gemm_f32(int form, const float* a, int64_t lda, const float* b, int64_t 
 namespace {
 
 // Batch rows per wave: all of a small batch, else 8 at a time (the weights'
-// rows then come from the caches again).
+// rows then come from the caches again). RW rows of the weight per wave and U
+// 16-byte loads a lane of each in flight: one pass over 256 U columns, so 768
+// for the products of d_model columns (RW 2, the head's many rows 4) and 1536
+// for those of d_inner columns (RW 1: few rows, more waves); with 8 batch rows
+// their registers leave 512. Chosen at 640 and 1432 columns, which one pass
+// then covers; wider rows take several passes, narrower ones leave lanes idle
+// (token us, native / module calls, batch 4: 384 and 856 columns 214 / 3179,
+// 1536 and 3472 479 / 2548).
 template <int KIND, int RW, int U>
 int launch_decode(const mhs::DecodeArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.rows + 4 * RW - 1) / (4 * RW))), block(256);

@@ -1,8 +1,9 @@
-"""Pre-tuned fp32 GEMM solutions for the TinyMamba train step on gfx950.
+"""Pre-tuned fp32 library GEMM solutions for the TinyMamba train step on gfx950.
 
-Outside the scan and the conv, a TinyMamba train step is fp32 GEMMs (the
-in/out projections, the merged dt/B/C projection of the fused inner block,
-and the 32768-way head). ``gemm_tuning_gfx950.csv``
+They serve the products that go to the library: the model with scan_impl
+'torch' and linear layers with hooks (the HIP path's in/out projections, merged
+dt/B/C projection and 32768-way head are the package's own products otherwise).
+``gemm_tuning_gfx950.csv``
 holds, for each GEMM shape of the 80M configuration (batch 16 x seq 512), the
 fastest of the rocBLAS / hipBLASLt fp32 solutions found by PyTorch's
 TunableOp on MI355X. ``use_tuned_gemms()`` loads it with tuning switched off,
@@ -53,6 +54,9 @@ def tune(out: Path, steps: int = 3, start: Path = TABLE) -> None:
     cfg = MambaConfig(vocab_size=32768, d_model=640, n_layers=12, d_ff=2560, max_seq_len=512,
                       d_state=16, d_conv=4, scan_impl="hip")
     model = TinyMamba(cfg).to(dev)
+    for m in model.modules():   # a hooked layer calls the library's product
+        if isinstance(m, torch.nn.Linear):
+            m.register_forward_hook(lambda mod, args, out: None)
     opt = torch.optim.AdamW(model.parameters(), lr=3e-4, fused=True)
     idx = torch.randint(0, cfg.vocab_size, (16, 513), device=dev)
     for step in range(steps):
