@@ -45,10 +45,10 @@ def block_params(block: nn.Module, x: torch.Tensor, strict: bool) -> Optional[tu
     """The block's parameters in mhs_block_weights' order where the native
     block takes them and x (batch, T, d_model), else None: plain modules
     without hooks or a forward of their own (strict: those too that the
-    block's fused path never calls),
-    fp32 contiguous 16-byte aligned parameters of the block's shapes, sizes
-    that are multiples of 4. The caller has checked the global hooks,
-    autocast, tracing and that x is an fp32 ROCm tensor."""
+    block's fused path never calls), plain fp32 contiguous 16-byte aligned
+    parameters of the block's shapes, sizes that are multiples of 4. The
+    caller has checked the global hooks, autocast, tracing and that x is an
+    fp32 ROCm tensor."""
     m, p = block._modules, block._parameters
     try:
         norm, in_proj, conv, dt_proj, b_proj, c_proj, out_proj = mods = (
@@ -171,10 +171,10 @@ class BlockHIP(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_x, g_out):
         x, xz, saved, *params = ctx.saved_tensors
+        x, xz, *params = (_restored(t, 16) for t in (x, xz, *params))
         if torch.is_grad_enabled():   # create_graph
             return _module_gradients(ctx, x, params, g_x, g_out)
         saved = _restored(saved, 256)
-        x, xz, *params = (_restored(t, 16) for t in (x, xz, *params))
         need = ctx.needs_input_grad
         if g_out is None:
             g_out = torch.zeros_like(x)

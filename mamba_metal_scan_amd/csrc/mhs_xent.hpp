@@ -168,8 +168,9 @@ xent_mean_kernel(const float* __restrict__ loss_rows, const long long* __restric
 }
 
 // HBM-bound: each logit read and each gradient written once (4096 x 50257:
-// 370 us with 4-byte accesses, 334 so, 4.9 TB/s, the rate of a copy). SAME: dlogits has logits' alignment
-// modulo 16 bytes; otherwise its elements are stored one by one.
+// 370 us with 4-byte accesses, 334 so, 4.9 TB/s, the rate of a copy). SAME:
+// dlogits has logits' alignment modulo 16 bytes; otherwise its elements are
+// stored one by one.
 template <bool SAME>
 __global__ void __launch_bounds__(kXentThreads)
 xent_bwd_kernel(const float* __restrict__ logits, const long long* __restrict__ targets,

@@ -30,8 +30,8 @@ def _layer(block: nn.Module, bc: dict, dev: torch.device, shapes: tuple, kinds: 
            conv_next: torch.Tensor) -> Optional[bytes]:
     """The block's mhs_decode_layer, or None where the native step does not
     take it: a module of another type, with hooks or with a forward of its
-    own, a weight that is not a plain fp32 parameter of its shape, a state or window that is not the
-    cache's own form."""
+    own, a weight that is not a plain fp32 parameter of its shape, a state or
+    window that is not the cache's own form."""
     m, p = block._modules, block._parameters
     try:
         norm, in_proj, conv, dt_proj, b_proj, c_proj, out_proj = mods = (
@@ -70,28 +70,37 @@ def batch_limit(d_model: int, d_inner: int, d_state: int, n_layers: int, vocab: 
 
     Its products pass over their weights, 512 columns at a time, again for
     every 8 rows, with VALU fmas: a layer (with its share of the head) costs
-    0.45 us a row and 0.136 us a row and million of weights so padded. The
-    module calls reuse tiles in the library's products: about 0.25 us a row
-    and 0.055 us a row and million weights, but on top of the launches, about
-    300 us a layer from Python and 70 to 170 us in a HIP graph. The line lies
-    where the native rows have used that up, with a margin: measured us a
-    token, native / modules, at the last batch won and the first lost, and
-    the line (vocabulary 32768; 200 at d_model 1024),
-      d_model, d_inner, layers  from Python                                in a graph
-      128, 272, 2        128: 450 / 705    256: 868 / 703    168    24: 114 / 136     32: 143 / 142     31
-      384, 856, 10       256: 2711 / 3409  512: 5313 / 3262  287   192: 2016 / 2153  256: 2702 / 2405   73
-      640, 1432, 12      128: 2632 / 4045  256: 5008 / 4045  167    96: 2031 / 2276  128: 2617 / 2454   38
-      1024, 2312, 24      64: 4393 / 7596  128: 8205 / 7996  123    64: 4363 / 4943   96: 6252 / 5809   30
-      1536, 3472, 8       32: 1633 / 2573   64: 2921 / 2712   53    24: 1302 / 1406   32: 1635 / 1588   13
+    about 0.7 us a row and 0.136 us a row and million of weights so padded, on
+    top of reading them once. The module calls reuse tiles in the library's
+    products, on top of their launches: 280 us and more a layer from Python; in
+    a HIP graph what those cost beyond the native token's, less what its
+    slower rows lose, comes to 100 us for every layer but one. us a token,
+    native / modules, at the last batch won and the first lost, and the line,
+    from Python and in a graph (vocabulary 32768; 200 at d_model 64, 1024 and
+    2048, 5000 at 516):
+      d_model 64, d_inner 88, 4 layers
+        188: 557 / 5020,  585: 1628 / 1340, 384;   64: 219 / 264,   188: 555 / 460,   102
+      128, 272, 2 layers
+        128: 450 / 705,   256: 868 / 703,   143;   24: 114 / 136,    32: 143 / 142,   26
+      384, 856, 10 layers
+        256: 2711 / 3409, 512: 5313 / 3262, 226;  192: 2016 / 2153, 256: 2702 / 2405, 73
+      516, 1152, 3 layers
+        206: 1000 / 1081,                   171;   64: 350 / 365,   206: 1006 / 619,  41
+      640, 1432, 12 layers
+        128: 2632 / 4045, 256: 5008 / 4045, 143;   96: 2031 / 2276, 128: 2617 / 2454, 47
+      1024, 2312, 24 layers
+        64: 4393 / 7596,  128: 8205 / 7996, 108;   64: 4363 / 4943,  96: 6252 / 5809, 38
+      1536, 3472, 8 layers
+        32: 1633 / 2573,   64: 2921 / 2712, 47;    24: 1302 / 1406,  32: 1635 / 1588, 16
+      2048, 4640, 4 layers
+        16: 717 / 1339,    36: 1457 / 1356, 31;    16: 718 / 804,    36: 1456 / 1227, 9
     Up to 8 rows the weights are read once, as any product must."""
     def padded(k: int) -> int:
         return (k + 511) // 512 * 512
-    wide = 2 * d_inner * padded(d_model) + (d_inner + 2 * d_state + d_model) * padded(d_inner)
-    wide += vocab * padded(d_model) / n_layers
-    plain_w = d_inner * (3 * d_model + d_inner + 2 * d_state) + vocab * d_model / n_layers
-    native = 0.45 + 0.136e-6 * wide
-    rows = 41.0 / (native - 0.25 - 0.055e-6 * plain_w) if captured else 280.0 / native
-    return max(8, int(rows))
+    weights = 2 * d_inner * padded(d_model) + (d_inner + 2 * d_state + d_model) * padded(d_inner)
+    weights += vocab * padded(d_model) / n_layers
+    budget = 100.0 - 100.0 / n_layers if captured else 280.0 - 0.6e-6 * weights
+    return max(8, int(budget / (0.7 + 0.136e-6 * weights)))
 
 
 def decode_step(model: nn.Module, x: torch.Tensor, cache: dict) -> Optional[torch.Tensor]:

@@ -56,9 +56,10 @@ def no_hooks(m: nn.Module) -> bool:
 
 def linear(mod: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """mod(x), through the HIP products where mod is a plain bias-free
-    nn.Linear (no subclass, no hooks, no forward of its own), x and its weight are fp32 on one ROCm
-    device outside autocast, and the product is large enough to be the faster
-    there (smaller ones keep the framework's call and its lower overhead)."""
+    nn.Linear (no subclass, no hooks, no forward of its own), x and its weight
+    are plain fp32 tensors on one ROCm device outside autocast, and the product
+    is large enough to be the faster there (smaller ones keep the framework's
+    call and its lower overhead)."""
     if (type(mod) is nn.Linear and mod.bias is None and _hip_device(x)
             and x.dtype == torch.float32 and not torch.is_autocast_enabled()):
         w = mod.weight
